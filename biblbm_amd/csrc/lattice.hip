@@ -439,6 +439,61 @@ bool zseg_ok(const bl_lattice_s* L, int B)
            (size_t)Q * (size_t)L->stride <= 0xffffffffull;
 }
 
+// The launch shape of a lattice that nobody tuned, by the bytes of its
+// populations against the 256 MiB last-level cache (the pass is bound by
+// memory; 4 GiB copy on the same card: 6.17 TB/s).  Ratios are against one
+// contiguous range of blocks per XCD without hints (order 1), even / odd
+// step, over cubes and channels of 64^3 to 384^3:
+//   fewer than 2^19 cells: order 1.  Chunks leave XCDs without work (64^3
+//     in chunks of 64: 0.96 / 0.94).
+//   in the cache: chunks of 256 blocks, so that the eight XCDs stream from
+//     nearby planes and a neighbour's row is read while it is still there:
+//     120 x 100 x 133 FP64 1.12 / 1.05, FP32 1.06 / 1.12, FP16s 1.15 / 1.25;
+//     hints lose there (0.6-0.9), they bypass the cache that holds it all.
+//   beyond it: chunks of 64 (FP64 201 x 199 x 181 1.16 / 1.07, FP32 1.13 /
+//     1.07, FP16s 1.12 / 0.97); even steps of FP64 and FP32 lattices whose
+//     planes start at multiples of 1 MiB, or beyond 2 GiB, stream past the
+//     cache instead, chunks of 16 (384^3 FP64 1.09 against 1.02, 256^3 FP32
+//     1.13 against 1.01: equally aligned planes compete for the same sets);
+//     FP64 odd steps take 128-cell z-segments, z-aligned and so whole-line
+//     streaming stores, where nz allows (256^3 1.08, 384^3 1.05).
+//   beyond it and carrying the velocity staging: the hints keep the vertex
+//     data, the force field and the staged velocities in the cache (512 x
+//     128 x 128 with 400 cells, FP32: even step 0.312 -> 0.235 ms, odd 0.315
+//     -> 0.27 ms in z-segments, -> 0.285 ms per cell; FP16s even 0.176 ->
+//     0.154 ms, odd no gain).
+void auto_launch(const bl_lattice_s* L, bool odd, bool emit, int& block, int& order, int& nt)
+{
+    constexpr size_t kCache = 256ull << 20;
+    const size_t plane = (size_t)L->stride * L->pop_bytes, bytes = Q * plane;
+    const bool half = L->storage == BL_STORE_F16S;
+    block = 256;
+    order = 1;
+    nt = 0;
+    if (L->ncell < (1L << 19)) return;
+    if (bytes <= kCache) {
+        order = 256;
+        return;
+    }
+    order = 64;
+    if (!odd) {
+        if (half) nt = emit ? 1 : 0;
+        else if (emit || plane % (1u << 20) == 0 || bytes > (2ull << 30)) {
+            order = 16;
+            nt = 1;
+        }
+        return;
+    }
+    if (half) return;
+    if ((emit || L->storage == BL_STORE_F64) && zseg_ok(L, 128) && !L->skip_inert) {
+        block = -128;
+        nt = 1;
+    } else if (emit) {
+        order = 16;
+        nt = 1;
+    }
+}
+
 static int force_mode(const bl_lattice_s* L)
 {
     if (L->tile_flags && L->force_field) return 2;
@@ -462,6 +517,7 @@ CollidePlan collide_plan(const bl_lattice_s* L)
     p.blk = L->block[par];
     v.xcd_remap = L->xcd_remap[par];
     p.nt = L->nontemporal[par];
+    if (p.blk == 0) auto_launch(L, p.odd, v.emit_u != nullptr, p.blk, v.xcd_remap, p.nt);
     if (p.blk < 0) {
         // the z-segment kernel steps every cell (its workgroups exchange
         // values through LDS), so it does not run with inert-cell skipping
@@ -1592,6 +1648,7 @@ int bl_lattice_get_launch(bl_lattice L, int parity, int out[3])
     out[0] = L->block[parity];
     out[1] = L->xcd_remap[parity];
     out[2] = L->nontemporal[parity];
+    if (out[0] == 0) auto_launch(L, parity == 1, false, out[0], out[1], out[2]);
     return BL_OK;
 }
 

@@ -69,9 +69,10 @@ struct bl_lattice_s {
 
     // launch shape of the collide-and-stream kernel per step parity (index 0
     // even, 1 odd): threads per block, XCD-aware block order, nontemporal
-    // population loads and stores (even step only; set by the tuner or a
-    // cached tuning result)
-    int block[2] = {256, 256};
+    // population loads and stores.  Block 0: nobody has fixed a shape, and
+    // each launch takes auto_launch's (set by the caller, the tuner or a
+    // cached tuning result otherwise)
+    int block[2] = {0, 0};
     int xcd_remap[2] = {1, 1};
     int nontemporal[2] = {0, 0};
 

@@ -175,7 +175,9 @@ int bl_lattice_set_launch(bl_lattice lat, int block, int xcd_remap);
  * a power of two (dealing segments as blocks), not BL_ORDER_ROWS.  Results
  * do not change. */
 int bl_lattice_set_launch_parity(bl_lattice lat, int parity, int block, int xcd_remap, int nontemporal);
-/* out = {block, xcd_remap, nontemporal} of one parity. */
+/* out = {block, xcd_remap, nontemporal} of one parity: as set, or, on a
+ * lattice that no call fixed or tuned, what a plain collide-and-stream
+ * takes by the lattice's size and storage. */
 int bl_lattice_get_launch(bl_lattice lat, int parity, int out[3]);
 /* HIP stream the lattice works on (hipStream_t), for event timing. */
 int bl_lattice_stream(bl_lattice lat, void **stream);
