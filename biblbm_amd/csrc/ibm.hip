@@ -1078,12 +1078,16 @@ __global__ void __launch_bounds__(256) k_interp(InterpArgs<R> a)
 // Every cell of a touched 4x4x4 tile sums g + phi phi phi F_k over the
 // tile's vertices in increasing vertex order, the order of the reference's
 // vertex loop (src/fsi/ImmersedBoundaryDynamics_forces.hh:53-85), and writes
-// its force; one lane per cell.  The tile's list is sorted first.  Then, 64
-// entries at a time, lane e loads entry e and forms its weights on the
-// tile's own 4 cells per axis (zero outside the stencil) and its force in
-// registers (all zero past the list's end); two halves of 32 go through LDS
-// in turn, and the cells walk each half in order, four entries per step,
-// with broadcast LDS reads.
+// its force.  The tile's list is sorted first.  Then, 64 entries at a time,
+// lane e loads entry e and forms its weights on the tile's own 4 cells per
+// axis (zero outside the stencil) and its force in registers (all zero past
+// the list's end); two halves of 32 go through LDS in turn.
+// The sum over a tile's entries is a matrix product: with the weights
+// separable, row (x, y) of A holds wx wy of entry k, column (component, z)
+// of B holds wz F, and the 16 x 12 result is the tile's force.  Four entries
+// are one 16x16x4 matrix instruction in the vertex real: per lane four LDS
+// reads and two multiplies, where a lane per cell took 24 reads and 24
+// fused multiply-adds for them (LDS reads bounded it).
 // One launch (k_spread) holds two kinds of workgroups:
 //   small: tiles with at most kSmallTile entries (the touched-tile list,
 //          skipping the others), one wave per tile, four independent waves
@@ -1097,7 +1101,30 @@ __global__ void __launch_bounds__(256) k_interp(InterpArgs<R> a)
 // Each clears the tile's count once done, so the next binning starts from
 // zero without a clearing pass.
 constexpr int kChunk = 32;
+// LDS row of a staged chunk: the 16 (row, entry) words that a matrix operand
+// reads at once, 4 rows of 4 entries, fall on 16 different banks
+constexpr int kChunkRow = kChunk + 4;
 constexpr int kSpreadWaves = 4;
+
+// c += A B over four entries: lane l gives A[l % 16][l / 16] and
+// B[l / 16][l % 16] and holds column l % 16 of c, four rows of it.  Rows are
+// the tile's (x, y), 4 x + y; columns 4 component + z.
+template <class R>
+struct TileSum;
+template <>
+struct TileSum<float> {
+    using V = float __attribute__((ext_vector_type(4)));
+    __device__ static V add(float a, float b, V c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+    __device__ static int x(int lane, int) { return lane >> 4; }
+    __device__ static int y(int, int r) { return r; }
+};
+template <>
+struct TileSum<double> {
+    using V = double __attribute__((ext_vector_type(4)));
+    __device__ static V add(double a, double b, V c) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0); }
+    __device__ static int x(int, int r) { return r; }
+    __device__ static int y(int lane, int) { return lane >> 4; }
+};
 
 // Orders the LDS accesses of one wave (a wave's LDS operations complete in
 // issue order; this keeps the compiler from moving them across).
@@ -1177,38 +1204,32 @@ __device__ __forceinline__ void entry_weights(const Grid& gd, int Sw, const int 
 }
 
 // Adds entries [0, cnt) of a staged half (cnt <= kChunk; the rows are zero
-// from cnt up to the next multiple of 4, so a padded entry adds nothing)
-// in entry order; the LDS reads of four entries are issued together.
+// from cnt to the half's end, so a padded entry adds nothing) in entry
+// order, 16 at a time.
 template <class R>
-__device__ __forceinline__ void chunk_sum(const R (*ew)[kChunk + 1], int cnt, int lx, int ly, int lz, R& a0, R& a1,
-                                          R& a2)
+__device__ __forceinline__ void chunk_sum(const R (*ew)[kChunkRow], int cnt, int lane, typename TileSum<R>::V& acc)
 {
-    for (int e = 0; e < cnt; e += 4) {
-        R w[4], f0[4], f1[4], f2[4];
+    const int k = lane >> 4, i = (lane >> 2) & 3, j = lane & 3;
+    const R *wx = ew[i] + k, *wy = ew[4 + j] + k, *wz = ew[8 + j] + k, *F = ew[12 + min(i, 2)] + k;
+    for (int e = 0; e < cnt; e += 16) {
+        R a[4], b[4];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            w[k] = (ew[lx][e + k] * ew[4 + ly][e + k]) * ew[8 + lz][e + k];
-            f0[k] = ew[12][e + k];
-            f1[k] = ew[13][e + k];
-            f2[k] = ew[14][e + k];
+        for (int q = 0; q < 4; ++q) {
+            a[q] = wx[e + 4 * q] * wy[e + 4 * q];
+            b[q] = wz[e + 4 * q] * F[e + 4 * q];
         }
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            a0 += w[k] * f0[k];
-            a1 += w[k] * f1[k];
-            a2 += w[k] * f2[k];
-        }
+        for (int q = 0; q < 4; ++q) acc = TileSum<R>::add(a[q], b[q], acc);
     }
 }
 
-// Sums the sorted entries [lo, hi) of a tile into a0..a2, 64 at a time;
-// key(e) gives the e-th sorted entry.
+// Adds the sorted entries [lo, hi) of a tile to acc, 64 at a time; key(e)
+// gives the e-th sorted entry.
 template <class R, class KeyOf>
 __device__ __forceinline__ void sum_entries(const Grid& gd, int Sw, const int org[3], int lo, int hi, KeyOf key,
                                             const int* __restrict__ base, const R* __restrict__ W,
                                             const R* __restrict__ vforce, const NearView<R>& nw,
-                                            R (*ew)[kChunk + 1], int lane, int lx, int ly, int lz, R& a0, R& a1,
-                                            R& a2)
+                                            R (*ew)[kChunkRow], int lane, typename TileSum<R>::V& acc)
 {
     for (int c0 = lo; c0 < hi; c0 += 64) {
         const int e = c0 + lane;
@@ -1224,7 +1245,7 @@ __device__ __forceinline__ void sum_entries(const Grid& gd, int Sw, const int or
 #pragma unroll
                 for (int r = 0; r < 15; ++r) ew[r][lane & (kChunk - 1)] = ev[r];
             wave_sync();
-            chunk_sum(ew, cnt, lx, ly, lz, a0, a1, a2);
+            chunk_sum<R>(ew, cnt, lane, acc);
             wave_sync();
         }
     }
@@ -1238,16 +1259,24 @@ __device__ __forceinline__ void tile_origin(const Grid& gd, int t, int org[3])
     org[2] = tz * kTile;
 }
 
-template <class FT, class R>
-__device__ __forceinline__ void store_cell(const LatView& lv, const Grid& gd, const int org[3], int lx, int ly,
-                                           int lz, R a0, R a1, R a2, FT* __restrict__ Fout)
+// The body force of a lane's column, the start of its sums.
+template <class R>
+__device__ __forceinline__ R column_start(const LatView& lv, int lane)
 {
-    const int x = org[0] + lx, y = org[1] + ly, z = org[2] + lz;
-    if (x < gd.n[0] && y < gd.n[1] && z < gd.n[2]) {
-        const long c = ((long)x * gd.n[1] + y) * gd.n[2] + z;
-        Fout[c] = (FT)a0;
-        Fout[lv.stride + c] = (FT)a1;
-        Fout[2 * lv.stride + c] = (FT)a2;
+    const int i = (lane >> 2) & 3;
+    return (R)(i == 0 ? lv.g[0] : (i == 1 ? lv.g[1] : lv.g[2]));
+}
+
+template <class FT, class R>
+__device__ __forceinline__ void store_tile(const LatView& lv, const Grid& gd, const int org[3], int lane,
+                                           typename TileSum<R>::V acc, FT* __restrict__ Fout)
+{
+    const int comp = (lane >> 2) & 3, z = org[2] + (lane & 3);
+    if (comp == 3 || z >= gd.n[2]) return;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int x = org[0] + TileSum<R>::x(lane, r), y = org[1] + TileSum<R>::y(lane, r);
+        if (x < gd.n[0] && y < gd.n[1]) Fout[comp * lv.stride + ((long)x * gd.n[1] + y) * gd.n[2] + z] = (FT)acc[r];
     }
 }
 
@@ -1277,7 +1306,7 @@ __device__ __forceinline__ int rank_in_run(const int* r, int key)
 }
 
 template <class FT, class R>
-__device__ __forceinline__ void spread_small(int blk, int nb, R (*ew_all)[15][kChunk + 1], const LatView& lv,
+__device__ __forceinline__ void spread_small(int blk, int nb, R (*ew_all)[15][kChunkRow], const LatView& lv,
                                              const Grid& gd, int Sw, const int* __restrict__ active,
                                              const int* __restrict__ nactive, int* __restrict__ count, int cap,
                                              const int* __restrict__ list, const int* __restrict__ base,
@@ -1285,10 +1314,9 @@ __device__ __forceinline__ void spread_small(int blk, int nb, R (*ew_all)[15][kC
                                              const NearView<R>& nw, FT* __restrict__ Fout)
 {
     const int wv = threadIdx.x >> 6;
-    R(*ew)[kChunk + 1] = ew_all[wv];
+    R(*ew)[kChunkRow] = ew_all[wv];
     const int na = *nactive;
     const int lane = threadIdx.x & 63;
-    const int lx = lane >> 4, ly = (lane >> 2) & 3, lz = lane & 3;
     const int stride = nb * kSpreadWaves;
     int a = blk * kSpreadWaves + wv;
     int t = a < na ? active[a] : 0;
@@ -1305,10 +1333,10 @@ __device__ __forceinline__ void spread_small(int blk, int nb, R (*ew_all)[15][kC
             const int key = wave_sort(lane < n ? raw : 0x7fffffff, lane);
             int org[3];
             tile_origin(gd, t, org);
-            R acc0 = (R)lv.g[0], acc1 = (R)lv.g[1], acc2 = (R)lv.g[2];
-            sum_entries<R>(gd, Sw, org, 0, n, [&](int) { return key; }, base, W, vforce, nw, ew, lane, lx, ly, lz,
-                           acc0, acc1, acc2);
-            store_cell(lv, gd, org, lx, ly, lz, acc0, acc1, acc2, Fout);
+            const R g = column_start<R>(lv, lane);
+            typename TileSum<R>::V acc = {g, g, g, g};
+            sum_entries<R>(gd, Sw, org, 0, n, [&](int) { return key; }, base, W, vforce, nw, ew, lane, acc);
+            store_tile<FT, R>(lv, gd, org, lane, acc, Fout);
             if (lane == 0) count[t] = 0;
         }
         a = a_next;
@@ -1317,8 +1345,8 @@ __device__ __forceinline__ void spread_small(int blk, int nb, R (*ew_all)[15][kC
 }
 
 template <class FT, class R>
-__device__ __forceinline__ void spread_big(int blk, int nb, int* keys, int* runs, R (*ew_all)[15][kChunk + 1],
-                                           R (*part)[3][64], const LatView& lv, const Grid& gd, int Sw,
+__device__ __forceinline__ void spread_big(int blk, int nb, int* keys, int* runs, R (*ew_all)[15][kChunkRow],
+                                           R (*part)[4][64], const LatView& lv, const Grid& gd, int Sw,
                                            const int* __restrict__ big, const int* __restrict__ nbig,
                                            int* __restrict__ count, int cap, const int* __restrict__ list,
                                            const int* __restrict__ base, const R* __restrict__ W,
@@ -1326,11 +1354,10 @@ __device__ __forceinline__ void spread_big(int blk, int nb, int* keys, int* runs
                                            FT* __restrict__ Fout)
 {
     const int wv = threadIdx.x >> 6;
-    R(*ew)[kChunk + 1] = ew_all[wv];
+    R(*ew)[kChunkRow] = ew_all[wv];
     const int nt = *nbig;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    const int lx = lane >> 4, ly = (lane >> 2) & 3, lz = lane & 3;
     for (int a = blk; a < nt; a += nb) {
         const int t = big[a];
         const int n = min(count[t], cap);  // a longer list was cut at binning and reported there
@@ -1375,21 +1402,19 @@ __device__ __forceinline__ void spread_big(int blk, int nb, int* keys, int* runs
         // wave w sums the contiguous range [lo, hi) of the sorted entries
         const int q = (n + kSpreadWaves - 1) / kSpreadWaves;
         const int lo = min(n, wv * q), hi = min(n, lo + q);
-        R acc0 = R(0), acc1 = R(0), acc2 = R(0);
-        sum_entries<R>(gd, Sw, org, lo, hi, [&](int k) { return keys[k]; }, base, W, vforce, nw, ew, lane, lx, ly,
-                       lz, acc0, acc1, acc2);
-        part[wv][0][lane] = acc0;
-        part[wv][1][lane] = acc1;
-        part[wv][2][lane] = acc2;
+        typename TileSum<R>::V acc = {R(0), R(0), R(0), R(0)};
+        sum_entries<R>(gd, Sw, org, lo, hi, [&](int k) { return keys[k]; }, base, W, vforce, nw, ew, lane, acc);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) part[wv][r][lane] = acc[r];
         __syncthreads();
         if (wv == 0) {
-            R s0 = (R)lv.g[0], s1 = (R)lv.g[1], s2 = (R)lv.g[2];
-            for (int w = 0; w < kSpreadWaves; ++w) {
-                s0 += part[w][0][lane];
-                s1 += part[w][1][lane];
-                s2 += part[w][2][lane];
-            }
-            store_cell(lv, gd, org, lx, ly, lz, s0, s1, s2, Fout);
+            const R g = column_start<R>(lv, lane);
+            acc = {g, g, g, g};
+#pragma unroll
+            for (int w = 0; w < kSpreadWaves; ++w)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[r] += part[w][r][lane];
+            store_tile<FT, R>(lv, gd, org, lane, acc, Fout);
             if (lane == 0) count[t] = 0;
         }
         __syncthreads();  // keys and partial sums are rewritten for the next tile
@@ -1419,8 +1444,8 @@ __device__ __forceinline__ void spread_body(int bx, int nbx, const SpreadArgs<R>
     using FT = typename Pop<S>::F;
     __shared__ int keys[kMaxList];
     __shared__ int runs[64 * kSpreadWaves];
-    __shared__ R ew_all[kSpreadWaves][15][kChunk + 1];
-    __shared__ R part[kSpreadWaves][3][64];
+    __shared__ R ew_all[kSpreadWaves][15][kChunkRow];
+    __shared__ R part[kSpreadWaves][4][64];
     if (bx < A.n_small)
         spread_small<FT, R>((int)ibm_block(bx, A.n_small, A.xcd), A.n_small, ew_all, A.lv, A.gd, A.Sw, A.active,
                             A.nactive, A.count, A.cap, A.list, A.base, A.W, A.vforce, A.nw, (FT*)A.Fout);
