@@ -37,8 +37,10 @@ namespace bl {
 namespace {
 
 constexpr int kTileCap = 512;      // list entries per 4x4x4 tile (stencils touching it)
-constexpr int kSmallTile = 64;     // tiles with more entries are spread by a whole workgroup
+constexpr int kSmallTile = 128;    // the most entries of a tile that one wave spreads (kSparseTile below)
+constexpr int kSparseTile = 64;    // the same where few tiles are touched: the others' waves are idle
 constexpr int kMaxList = kTileCap; // entries the spreading kernel sorts in LDS
+static_assert(kMaxList >= 4 * kSmallTile, "four waves of small tiles order their keys there");
 
 // ------------------------------------------------------------- helpers
 // Vertex data (positions, velocities, forces, element forces, stencil
@@ -47,17 +49,22 @@ constexpr int kMaxList = kTileCap; // entries the spreading kernel sorts in LDS
 // geometry, per-particle area / volume / centroid reductions and the
 // conservation sums stay FP64 in both.
 
-// Delta kernels (src/fsi/Dirac.h:23-66,74-101), 1-D factor.
+// Delta kernels (src/fsi/Dirac.h:23-66,74-101), 1-D factor; the branch is
+// taken on the square root's argument, so that a lane forms one root.
 template <class R>
 __device__ __forceinline__ R dirac(int kernel, R x)
 {
     const R dx = fabs(x);
-    if (kernel == BL_KERNEL_ROMA)
-        return (R(1.0) / R(6.0)) * (dx > R(0.5) ? (R(5.0) - R(3) * dx - sqrt(-R(3) * (R(1) - dx) * (R(1) - dx) + R(1)))
-                                                : R(2.0) * (R(1) + sqrt(R(1) - R(3) * dx * dx)));
-    if (kernel == BL_KERNEL_PESKIN)
-        return R(0.125) * (dx <= R(1) ? (R(3) - R(2) * dx + sqrt(R(1) + R(4) * dx * (R(1) - dx)))
-                                      : (R(5) - R(2) * dx - sqrt(-R(7) + R(4) * dx * (R(3) - dx))));
+    if (kernel == BL_KERNEL_ROMA) {
+        const bool far = dx > R(0.5);
+        const R q = sqrt(far ? -R(3) * (R(1) - dx) * (R(1) - dx) + R(1) : R(1) - R(3) * dx * dx);
+        return (R(1.0) / R(6.0)) * (far ? (R(5.0) - R(3) * dx - q) : R(2.0) * (R(1) + q));
+    }
+    if (kernel == BL_KERNEL_PESKIN) {
+        const bool near = dx <= R(1);
+        const R q = sqrt(near ? R(1) + R(4) * dx * (R(1) - dx) : -R(7) + R(4) * dx * (R(3) - dx));
+        return R(0.125) * (near ? (R(3) - R(2) * dx + q) : (R(5) - R(2) * dx - q));
+    }
     return R(1.) - fabs(x);
 }
 
@@ -155,9 +162,15 @@ struct AxisTiles {
 __device__ __forceinline__ AxisTiles axis_tiles(int bw, int S, int n, int per)
 {
     AxisTiles r;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const int node = k < S ? node_at(bw, k, n, per) : -1;
+    if (bw >= 0 && bw + S <= n) {  // nearly every stencil: no face inside it
+        r.t0 = bw >> 2;
+        r.t1 = (bw + S - 1) >> 2;
+        r.m = r.t1 != r.t0 ? 2 : 1;
+        return r;
+    }
+#pragma unroll 1
+    for (int k = 0; k < S; ++k) {
+        const int node = node_at(bw, k, n, per);
         const int t = node >> 2;
         const bool fresh = node >= 0 && t != r.t0 && t != r.t1 && t != r.t2;
         if (fresh) {
@@ -170,13 +183,72 @@ __device__ __forceinline__ AxisTiles axis_tiles(int bw, int S, int n, int per)
     return r;
 }
 
+// First node of a stencil of half support h (unwrapped), and the same
+// wrapped on a periodic axis (node_at's base).
+template <class R>
+__device__ __forceinline__ int stencil_first(R x, R h) { return (int)ceil(x - h); }
+
+__device__ __forceinline__ int stencil_base(int first, int n, int per)
+{
+    if (!per || (first >= 0 && first < n)) return first;
+    const int b = first % n;
+    return b < 0 ? b + n : b;
+}
+
+// The stencil's weights along one axis, of the nodes first .. first + 3
+// (zero past the support).  The nodes' distances are r + 1, r, 1 - r, 2 - r
+// (Peskin) and 1 + r, r, 1 - r (Roma) with r = x - (first + 1), and phi's
+// square roots at all of them are the one at r: 1 + 4 r (1 - r) and
+// 1 - 3 r^2.  In registers by name: an indexed array here went to scratch.
+template <class R>
+struct W4 {
+    R w0, w1, w2, w3;
+};
+
+template <class R>
+__device__ __forceinline__ W4<R> axis_weights(int kernel, R x, int first)
+{
+    const R r = x - (R)(first + 1);
+    if (kernel == BL_KERNEL_PESKIN) {
+        const R q = sqrt(R(1) + R(4) * r * (R(1) - r));
+        const R a = R(3) - R(2) * r, b = R(1) + R(2) * r;
+        return {R(0.125) * (a - q), R(0.125) * (a + q), R(0.125) * (b + q), R(0.125) * (b - q)};
+    }
+    if (kernel == BL_KERNEL_ROMA) {
+        const R q = sqrt(R(1) - R(3) * r * r);
+        constexpr R s = R(1.0) / R(6.0);
+        return {s * (R(2) - R(3) * r - q), (R(1.0) / R(3.0)) * (R(1) + q), s * (R(2) + R(3) * r - q), R(0)};
+    }
+    return {-r, R(1) + r, R(0), R(0)};
+}
+
+// The weights on four consecutive nodes, `shift` nodes past the stencil's
+// first one (-3 .. 3; zero where the stencil does not reach): three
+// conditional shifts by 4, 2 and 1.
+template <class R>
+__device__ __forceinline__ void shifted(const W4<R>& w, int shift, R o[4])
+{
+    const int t = shift + 3;
+    const bool b4 = t & 4, b2 = t & 2, b1 = t & 1;
+    const R z = R(0);
+    const R y0 = b4 ? w.w1 : z, y1 = b4 ? w.w2 : z, y2 = b4 ? w.w3 : z, y3 = b4 ? z : w.w0, y4 = b4 ? z : w.w1,
+            y5 = b4 ? z : w.w2, y6 = b4 ? z : w.w3;
+    const R z0 = b2 ? y2 : y0, z1 = b2 ? y3 : y1, z2 = b2 ? y4 : y2, z3 = b2 ? y5 : y3, z4 = b2 ? y6 : y4;
+    o[0] = b1 ? z1 : z0;
+    o[1] = b1 ? z2 : z1;
+    o[2] = b1 ? z3 : z2;
+    o[3] = b1 ? z4 : z3;
+}
+
 // Tiles touched by a vertex's stencil: the product of the per-axis sets.
 struct StencilTiles {
     AxisTiles ax[3];
-    __device__ __forceinline__ void init(const Grid& gd, int S, const int* b)
+    template <class R>
+    __device__ __forceinline__ void init(const Grid& gd, int S, R h, const R x[3])
     {
 #pragma unroll
-        for (int a = 0; a < 3; ++a) ax[a] = axis_tiles(b[a], S, gd.n[a], gd.per[a]);
+        for (int a = 0; a < 3; ++a)
+            ax[a] = axis_tiles(stencil_base(stencil_first(x[a], h), gd.n[a], gd.per[a]), S, gd.n[a], gd.per[a]);
     }
     // tile (i, j, k) of the product, or -1 past the per-axis counts
     __device__ __forceinline__ int at(const Grid& gd, int i, int j, int k) const
@@ -184,6 +256,7 @@ struct StencilTiles {
         if (i >= ax[0].m || j >= ax[1].m || k >= ax[2].m) return -1;
         return (ax[0].get(i) * gd.nt[1] + ax[1].get(j)) * gd.nt[2] + ax[2].get(k);
     }
+    __device__ __forceinline__ bool wide() const { return ax[0].m > 2 || ax[1].m > 2 || ax[2].m > 2; }
 };
 
 // Neighbouring vertices of a membrane touch the same few tiles, so a
@@ -191,7 +264,7 @@ struct StencilTiles {
 // (open addressing, linear probing) and then issues one global atomic per
 // distinct tile.  A pair whose tile finds the table full goes straight to
 // the global counter; counts stay exact either way.
-constexpr int kHashBits = 9;  // 512 slots: a workgroup's 256 vertices touch a few dozen tiles
+constexpr int kHashBits = 9;  // 512 slots: a workgroup's 256 vertices touch at most some two hundred tiles
 constexpr int kHash = 1 << kHashBits;
 
 __device__ __forceinline__ int hash_insert(int* keys, int t)
@@ -203,29 +276,6 @@ __device__ __forceinline__ int hash_insert(int* keys, int t)
         h = (h + 1) & (kHash - 1);
     }
     return -1;
-}
-
-// slot of a tile inserted earlier in the same workgroup, -1 if its insert
-// found the table full (then it was never inserted)
-__device__ __forceinline__ int hash_find(const int* keys, int t)
-{
-    unsigned h = ((unsigned)t * 2654435761u) >> (32 - kHashBits);
-    for (int probe = 0; probe < kHash; ++probe) {
-        const int k = keys[h];
-        if (k == t) return (int)h;
-        if (k == -1) return -1;
-        h = (h + 1) & (kHash - 1);
-    }
-    return -1;
-}
-
-__device__ __forceinline__ void hash_clear(int* keys, int* a, int* b)
-{
-    for (int i = threadIdx.x; i < kHash; i += blockDim.x) {
-        keys[i] = -1;
-        a[i] = 0;
-        if (b) b[i] = 0;
-    }
 }
 
 // Readies list `act` (length *na) / flag buffer `flags` for a binning:
@@ -282,8 +332,6 @@ struct NearView {
     int on = 0;                      // a boundary is set
     unsigned char* near = nullptr;   // per vertex: near-wall
     R* blend = nullptr;              // per vertex: distance - half support
-    int* base_t = nullptr;           // per vertex: top-hat stencil base (3)
-    R* W_t = nullptr;                // per vertex: top-hat weights (2 per axis)
 };
 
 // The first pair that reaches a tile (outside a workgroup's table) lists it
@@ -294,71 +342,27 @@ __device__ __forceinline__ void touch_tile(int t, int* act, int* na, unsigned ch
     flags[t] = 1;
 }
 
-__device__ __forceinline__ void count_tiles(const StencilTiles& st, const Grid& gd, int* keys, int* cnt)
-{
-#pragma unroll 1
-    for (int i = 0; i < st.ax[0].m; ++i)
-#pragma unroll 1
-        for (int j = 0; j < st.ax[1].m; ++j)
-#pragma unroll 1
-            for (int k = 0; k < st.ax[2].m; ++k) {
-                const int sl = hash_insert(keys, st.at(gd, i, j, k));
-                if (sl >= 0) atomicAdd(&cnt[sl], 1);
-            }
-}
+// Binning in one pass: the tiles each vertex's stencil touches, and every
+// (tile, vertex) pair written into the tile's fixed-capacity list (entry
+// values as described at kNearKey; a near-wall vertex also gets its blend
+// weight and the tiles of its top-hat stencil).  The vertex's position is
+// copied to `vp` (x, y, z, 1; all zero for a vertex that takes no part):
+// spreading and interpolation form the stencil weights from that copy, one
+// aligned load, while the advection moves the vertex itself.  Eight lanes
+// take a vertex, one per tile of the 2 x 2 x 2 product.  Per workgroup the
+// pairs are counted per distinct tile in LDS (the count at its insert is a
+// pair's place in the workgroup's run), one global atomic per tile reserves
+// the run.  The order within a list is whatever the atomics give; spreading
+// sorts.  The add that takes a tile past kSmallTile entries appends it to
+// the big-tile list.
+// Bound by latency on one cell and by instructions on many.  A thread per
+// vertex walking its tiles twice, with the weights stored (60 B a vertex in
+// FP32), took 16 us beside the element forces for 642 vertices and 99 us for
+// 400 800; this takes 7.1 and 87 us.
+constexpr int kBinLanes = 8;
+constexpr long kManyVertices = 65536;
+constexpr int kBinMany = 8;  // vertices per lane group from kManyVertices on: fewer distinct tiles per pair
 
-__device__ __forceinline__ void fill_tiles(const StencilTiles& st, const Grid& gd, int entry, const int* keys,
-                                           const int* cnt, int* rank, int* count, int* list, int cap, int* act,
-                                           int* na, unsigned char* flags, int* status, int* pairs, int* big,
-                                           int* nbig)
-{
-#pragma unroll 1
-    for (int i = 0; i < st.ax[0].m; ++i)
-#pragma unroll 1
-        for (int j = 0; j < st.ax[1].m; ++j)
-#pragma unroll 1
-            for (int k = 0; k < st.ax[2].m; ++k) {
-                const int tt = st.at(gd, i, j, k);
-                const int sl = hash_find(keys, tt);
-                int slot;
-                if (sl >= 0) {
-                    slot = cnt[sl] + atomicAdd(&rank[sl], 1);
-                } else {  // the workgroup's table was full for this tile
-                    slot = atomicAdd(&count[tt], 1);
-                    if (slot == 0) touch_tile(tt, act, na, flags);
-                    if (slot == kSmallTile) big[atomicAdd(nbig, 1)] = tt;
-                    atomicAdd(pairs, 1);
-                    if (slot >= cap) atomicOr(&status[2], 1);
-                }
-                if (slot < cap) list[(long)tt * cap + slot] = entry;
-            }
-}
-
-// Support-box base (wrapped on periodic axes) and the S weights of one axis.
-template <class R>
-__device__ __forceinline__ int axis_stencil(int kernel, int S, R h, R x, int n, int per, R* w)
-{
-    const int raw = (int)ceil(x - h);
-#pragma unroll 1
-    for (int k = 0; k < 4; ++k)
-        if (k < S) w[k] = dirac<R>(kernel, (R)(raw + k) - x);
-    int bw = raw;
-    if (per) {
-        bw = raw % n;
-        if (bw < 0) bw += n;
-    }
-    return bw;
-}
-
-// Binning in one pass: stencil base and 1-D weights per vertex, the tiles
-// its stencil touches, and every (tile, vertex) pair written into the
-// tile's fixed-capacity list (entry values as described at kNearKey; a
-// near-wall vertex also gets its blend weight, top-hat base and weights and
-// the tiles of its top-hat stencil).  Per workgroup the pairs are counted
-// per distinct tile in LDS, one global atomic per tile reserves the
-// workgroup's run, and the slots inside the run come from LDS.  The order
-// within a list is whatever the atomics give; spreading sorts.  The add that
-// takes a tile past kSmallTile entries appends it to the big-tile list.
 template <class R>
 struct BinArgs {
     Grid gd;
@@ -366,106 +370,140 @@ struct BinArgs {
     double h;
     long NV;
     const R* pos;
-    int* base;
-    R* W;
+    Vel4<R>* vp;
     int *count, *list;
     int cap;
     int *act, *na;
     unsigned char* flags;
     int *status, *pairs, *big, *nbig;
+    int small;  // entries past which a tile joins the big-tile list
     NearView<R> nw;
     int xcd;  // workgroup order (ibm_block)
 };
 
+// One pair past the workgroup's table, straight into the tile's list.
 template <class R>
+__device__ __forceinline__ void put_pair(const BinArgs<R>& A, int t, int entry)
+{
+    const int slot = atomicAdd(&A.count[t], 1);
+    if (slot == 0) touch_tile(t, A.act, A.na, A.flags);
+    if (slot == A.small) A.big[atomicAdd(A.nbig, 1)] = t;
+    atomicAdd(A.pairs, 1);
+    if (slot >= A.cap) atomicOr(&A.status[2], 1);
+    else A.list[(long)t * A.cap + slot] = entry;
+}
+
+// This lane's tile of a stencil counted in the table: slot and rank there
+// (slot * 65536 + rank), or -1 when there is nothing left to place.
+template <class R>
+__device__ __forceinline__ int count_pair(const BinArgs<R>& A, const StencilTiles& st, int r, int entry, int* keys,
+                                          int* cnt)
+{
+    // tiles past the 2 x 2 x 2 product: a third one on an axis (a wrap at a
+    // size that is no multiple of 4), and a full table
+    int direct = -1;
+    const int t = st.at(A.gd, r >> 2, (r >> 1) & 1, r & 1);
+    int code = -1;
+    if (t >= 0) {
+        const int sl = hash_insert(keys, t);
+        if (sl >= 0) code = (sl << 16) + atomicAdd(&cnt[sl], 1);
+        else direct = t;
+    }
+    if (direct >= 0 || st.wide()) {
+#pragma unroll 1
+        for (int q = r - kBinLanes; q < 27; q += kBinLanes) {
+            const int i = q / 9, j = q / 3 % 3, k = q % 3;
+            int tq = direct;
+            direct = -1;
+            if (q >= 0) tq = i == 2 || j == 2 || k == 2 ? st.at(A.gd, i, j, k) : -1;
+            if (tq >= 0) put_pair(A, tq, entry);
+        }
+    }
+    return code;
+}
+
+template <class R>
+__device__ __forceinline__ void place_pair(const BinArgs<R>& A, int code, int entry, const int* keys, const int* cnt)
+{
+    if (code < 0) return;
+    const int sl = code >> 16, slot = cnt[sl] + (code & 0xffff);
+    if (slot < A.cap) A.list[(long)keys[sl] * A.cap + slot] = entry;
+}
+
+// ITER vertices per group of lanes, NEAR: a boundary is set (then ITER is 1
+// and a vertex's top-hat entry takes a second code).
+template <class R, bool NEAR, int ITER>
 __device__ __forceinline__ void bin_body(long bx, const BinArgs<R>& A)
 {
-    const Grid& gd = A.gd;
-    const int kernel = A.kernel, S = A.S, cap = A.cap;
-    const R h = (R)A.h;
-    const long NV = A.NV;
-    const R* __restrict__ pos = A.pos;
-    int* __restrict__ base = A.base;
-    R* __restrict__ W = A.W;
-    int* __restrict__ count = A.count;
-    int* __restrict__ list = A.list;
-    int* __restrict__ act = A.act;
-    int* __restrict__ na = A.na;
-    unsigned char* __restrict__ flags = A.flags;
-    int* __restrict__ status = A.status;
-    int* __restrict__ pairs = A.pairs;
-    int* __restrict__ big = A.big;
-    int* __restrict__ nbig = A.nbig;
-    const NearView<R>& nw = A.nw;
     __shared__ int keys[kHash];
-    __shared__ int cnt[kHash];  // pairs per slot, then the slot's first index in the tile's list
-    __shared__ int rank[kHash];
+    __shared__ int cnt[kHash];    // pairs per slot, then the run's first index in the tile's list
     __shared__ int fresh[kHash];  // tiles this workgroup reached first
     __shared__ int occ[kHash];    // occupied slots, compacted
+    __shared__ int codes[ITER > 1 ? ITER * 256 : 1];
     __shared__ int n_fresh, n_pairs, fresh_base, n_occ;
-    hash_clear(keys, cnt, rank);
+    for (int i = threadIdx.x; i < kHash; i += blockDim.x) {
+        keys[i] = -1;
+        cnt[i] = 0;
+    }
     if (threadIdx.x == 0) {
         n_fresh = 0;
         n_pairs = 0;
         n_occ = 0;
     }
+    const int r = threadIdx.x & (kBinLanes - 1);
+    const int vpw = blockDim.x / kBinLanes;
+    const long v0 = bx * vpw * ITER + threadIdx.x / kBinLanes;
+    const NearView<R>& nw = A.nw;
+    const R* __restrict__ pos = A.pos;
+    int code = -1, codet = -1, e0 = -1, e1 = -1;
+    // the next vertex's position loads while this one is binned
+    R nx[3];
+    for (int a = 0; a < 3; ++a) nx[a] = pos[3 * min(v0, A.NV - 1) + a];
     __syncthreads();
-    const long v = bx * blockDim.x + threadIdx.x;
-    StencilTiles st, stt;
-    int e0 = -1, e1 = -1;  // list entries of the kernel part and the top-hat part (-1: none)
-    // a vertex whose position is not finite (a membrane that blew up) or
-    // absurdly far off touches no tile: zero weights at base 0, reported
-    bool off = false;
-    if (v < NV)
-        for (int a = 0; a < 3; ++a) off = off || !(fabs(pos[3 * v + a]) < R(1e9));
-    if (v < NV && off) {
-        for (int a = 0; a < 3; ++a) {
-            base[3 * v + a] = 0;
-            for (int k = 0; k < 4; ++k) W[12 * v + 4 * a + k] = R(0.0);
+#pragma unroll 1
+    for (int it = 0; it < ITER; ++it) {
+        const long v = v0 + it * vpw;
+        const R x[3] = {nx[0], nx[1], nx[2]};
+        if (it + 1 < ITER) {
+            const long vn = min(v + vpw, A.NV - 1);
+            for (int a = 0; a < 3; ++a) nx[a] = pos[3 * vn + a];
         }
-        if (nw.on) {
-            nw.near[v] = 0;
-            nw.blend[v] = R(1.0);
-        }
-        atomicOr(&status[2], 4);
-    }
-    if (v < NV && !off) {
-        int b[3];
-        for (int a = 0; a < 3; ++a) {
-            R w[4] = {R(0.0), R(0.0), R(0.0), R(0.0)};
-            b[a] = axis_stencil<R>(kernel, S, h, pos[3 * v + a], gd.n[a], gd.per[a], w);
-            base[3 * v + a] = b[a];
-            for (int k = 0; k < 4; ++k) W[12 * v + 4 * a + k] = w[k];
-        }
-        st.init(gd, S, b);
-        e0 = (int)v;
-        if (nw.on) {
-            // the wall distance in FP64 (the boundary's own arithmetic)
-            const double p[3] = {(double)pos[3 * v], (double)pos[3 * v + 1], (double)pos[3 * v + 2]};
-            const bool nr = bnd_less_than(nw.b, p, A.h + 1.);
-            const R wb = (R)(bnd_distance(nw.b, p) - A.h);
-            nw.near[v] = nr;
-            nw.blend[v] = wb;
-            if (nr) {
-                e0 = wb > R(0) ? (kNearKey | (int)(2 * v)) : -1;
-                if (wb < R(1)) {
-                    int bt[3];
-                    for (int a = 0; a < 3; ++a) {
-                        R w[4];
-                        bt[a] = axis_stencil<R>(BL_KERNEL_TOPHAT, 2, R(1.0), pos[3 * v + a], gd.n[a], gd.per[a], w);
-                        nw.base_t[3 * v + a] = bt[a];
-                        nw.W_t[6 * v + 2 * a] = w[0];
-                        nw.W_t[6 * v + 2 * a + 1] = w[1];
+        code = e0 = -1;
+        if (v < A.NV) {
+            // a vertex whose position is not finite (a membrane that blew
+            // up) or absurdly far off touches no tile and is reported
+            const bool off = !(fabs(x[0]) < R(1e9)) || !(fabs(x[1]) < R(1e9)) || !(fabs(x[2]) < R(1e9));
+            if (r == 0) {
+                A.vp[v] = off ? Vel4<R>{R(0), R(0), R(0), R(0)} : Vel4<R>{x[0], x[1], x[2], R(1)};
+                if (off) atomicOr(&A.status[2], 4);
+            }
+            if (!off) e0 = (int)v;
+            if (NEAR) {
+                // the wall distance in FP64 (the boundary's own arithmetic)
+                const double p[3] = {(double)x[0], (double)x[1], (double)x[2]};
+                const bool nr = !off && bnd_less_than(nw.b, p, A.h + 1.);
+                const R wb = off ? R(1.0) : (R)(bnd_distance(nw.b, p) - A.h);
+                if (r == 0) {
+                    nw.near[v] = nr;
+                    nw.blend[v] = wb;
+                }
+                if (nr) {
+                    e0 = wb > R(0) ? (kNearKey | (int)(2 * v)) : -1;
+                    if (wb < R(1)) {
+                        e1 = kNearKey | (int)(2 * v + 1);
+                        StencilTiles stt;
+                        stt.init(A.gd, 2, R(1.0), x);
+                        codet = count_pair(A, stt, r, e1, keys, cnt);
                     }
-                    stt.init(gd, 2, bt);
-                    e1 = kNearKey | (int)(2 * v + 1);
                 }
             }
+            if (e0 >= 0) {
+                StencilTiles st;
+                st.init(A.gd, A.S, (R)A.h, x);
+                code = count_pair(A, st, r, e0, keys, cnt);
+            }
         }
-        // runtime loops: the kernel runs once per launch on few workgroups,
-        // so compact code (instruction fetch) beats unrolling
-        if (e0 >= 0) count_tiles(st, gd, keys, cnt);
-        if (e1 >= 0) count_tiles(stt, gd, keys, cnt);
+        if (ITER > 1) codes[it * blockDim.x + threadIdx.x] = code;
     }
     __syncthreads();
     // one global atomic per distinct tile; the occupied slots are compacted
@@ -477,35 +515,55 @@ __device__ __forceinline__ void bin_body(long bx, const BinArgs<R>& A)
         const int i = occ[k];
         const int c = cnt[i];
         const int t = keys[i];
-        const int old = atomicAdd(&count[t], c);
+        const int old = atomicAdd(&A.count[t], c);
         cnt[i] = old;
         if (old == 0) fresh[atomicAdd(&n_fresh, 1)] = t;
-        if (old <= kSmallTile && old + c > kSmallTile) big[atomicAdd(nbig, 1)] = t;
+        if (old <= A.small && old + c > A.small) A.big[atomicAdd(A.nbig, 1)] = t;
         atomicAdd(&n_pairs, c);
-        if (old + c > cap) atomicOr(&status[2], 1);
+        if (old + c > A.cap) atomicOr(&A.status[2], 1);
     }
     __syncthreads();
     // the touched-list reservation is issued before the list fill and its
     // result read after it, so the two round trips overlap
     int fb = 0;
     if (threadIdx.x == 0) {
-        if (n_fresh) fb = atomicAdd(na, n_fresh);
-        if (n_pairs) atomicAdd(pairs, n_pairs);
+        if (n_fresh) fb = atomicAdd(A.na, n_fresh);
+        if (n_pairs) atomicAdd(A.pairs, n_pairs);
     }
-    if (e0 >= 0) fill_tiles(st, gd, e0, keys, cnt, rank, count, list, cap, act, na, flags, status, pairs, big, nbig);
-    if (e1 >= 0) fill_tiles(stt, gd, e1, keys, cnt, rank, count, list, cap, act, na, flags, status, pairs, big, nbig);
+    if (ITER > 1) {
+#pragma unroll 4
+        for (int it = 0; it < ITER; ++it)
+            place_pair(A, codes[it * blockDim.x + threadIdx.x], (int)(v0 + it * vpw), keys, cnt);
+    } else {
+        place_pair(A, code, e0, keys, cnt);
+        if (NEAR) place_pair(A, codet, e1, keys, cnt);
+    }
     if (threadIdx.x == 0) fresh_base = fb;
     __syncthreads();
     for (int i = threadIdx.x; i < n_fresh; i += blockDim.x) {
-        act[fresh_base + i] = fresh[i];
-        flags[fresh[i]] = 1;
+        A.act[fresh_base + i] = fresh[i];
+        A.flags[fresh[i]] = 1;
     }
+}
+
+// A binning workgroup of one vertex per lane group.
+template <class R>
+__device__ __forceinline__ void bin_one(long bx, const BinArgs<R>& A)
+{
+    if (A.nw.on) bin_body<R, true, 1>(bx, A);
+    else bin_body<R, false, 1>(bx, A);
 }
 
 template <class R>
 __global__ void __launch_bounds__(256) k_bin(BinArgs<R> a)
 {
-    bin_body<R>(ibm_block(blockIdx.x, gridDim.x, a.xcd), a);
+    bin_one<R>(ibm_block(blockIdx.x, gridDim.x, a.xcd), a);
+}
+
+template <class R>
+__global__ void __launch_bounds__(256) k_bin_many(BinArgs<R> a)
+{
+    bin_body<R, false, kBinMany>(ibm_block(blockIdx.x, gridDim.x, a.xcd), a);
 }
 
 __global__ void k_clear_bins(int* count, long n)
@@ -961,9 +1019,10 @@ template <class R>
 struct InterpArgs {
     Grid gd;
     long NV;
-    const int* base;
-    const R* W;
-    const void* ut;  // Vel4<C>
+    int kernel;
+    double h;
+    const Vel4<R>* vp;  // the binning's position copies
+    const void* ut;     // Vel4<C>
     R *vel, *pos;
     ListReset lr;
     NearView<R> nw;
@@ -975,8 +1034,6 @@ __device__ __forceinline__ void interp_body(long bx, int nbx, const InterpArgs<R
 {
     const Grid& gd = A.gd;
     const long NV = A.NV;
-    const int* __restrict__ base = A.base;
-    const R* __restrict__ W = A.W;
     const Vel4<C>* __restrict__ ut = (const Vel4<C>*)A.ut;
     R* __restrict__ vel = A.vel;
     R* __restrict__ pos = A.pos;
@@ -989,18 +1046,34 @@ __device__ __forceinline__ void interp_body(long bx, int nbx, const InterpArgs<R
     const int r = (int)(gid % LPV);
     const int j = r / LA, k = r % LA;
     R a0 = R(0), a1 = R(0), a2 = R(0);
-    if (v < NV && j < SW && k < SW) {
-        const int yj = node_at(base[3 * v + 1], j, gd.n[1], gd.per[1]);
-        const int zk = node_at(base[3 * v + 2], k, gd.n[2], gd.per[2]);
+    const Vel4<R> P = v < NV ? A.vp[v] : Vel4<R>{R(0), R(0), R(0), R(0)};
+    const R h = (R)A.h;
+    const int fx = stencil_first(P.x, h), fy = stencil_first(P.y, h), fz = stencil_first(P.z, h);
+    // the stencil's weights: a lane of the group forms one of the twelve and
+    // the group shares them (a top-hat weight costs less than the exchange)
+    R wx[SW], wy, wz;
+    if (SW == 2) {
+#pragma unroll
+        for (int i = 0; i < SW; ++i) wx[i] = dirac<R>(A.kernel, (R)(fx + i) - P.x);
+        wy = dirac<R>(A.kernel, (R)(fy + j) - P.y);
+        wz = dirac<R>(A.kernel, (R)(fz + k) - P.z);
+    } else {
+        const R mine = dirac<R>(A.kernel, (j == 0 ? (R)(fx + k) - P.x : (j == 1 ? (R)(fy + k) - P.y : (R)(fz + k) - P.z)));
+#pragma unroll
+        for (int i = 0; i < SW; ++i) wx[i] = __shfl(mine, i, LPV);
+        wy = __shfl(mine, 4 + j, LPV);
+        wz = __shfl(mine, 8 + k, LPV);
+    }
+    if (P.w != R(0) && j < SW && k < SW) {
+        const int yj = node_at(stencil_base(fy, gd.n[1], gd.per[1]), j, gd.n[1], gd.per[1]);
+        const int zk = node_at(stencil_base(fz, gd.n[2], gd.per[2]), k, gd.n[2], gd.per[2]);
         if (yj >= 0 && zk >= 0) {
-            const R* Wv = W + 12 * v;
-            const R wy = Wv[4 + j], wz = Wv[8 + k];
-            const int bx = base[3 * v];
+            const int b0 = stencil_base(fx, gd.n[0], gd.per[0]);
 #pragma unroll
             for (int i = 0; i < SW; ++i) {
-                const int xi = node_at(bx, i, gd.n[0], gd.per[0]);
+                const int xi = node_at(b0, i, gd.n[0], gd.per[0]);
                 if (xi < 0) continue;
-                const R w = (Wv[i] * wy) * wz;
+                const R w = (wx[i] * wy) * wz;
                 const Vel4<C> u = ut[((size_t)xi * gd.n[1] + yj) * gd.n[2] + zk];
                 a0 += w * (R)u.x;
                 a1 += w * (R)u.y;
@@ -1018,16 +1091,16 @@ __device__ __forceinline__ void interp_body(long bx, int nbx, const InterpArgs<R
         const R wb = nw.blend[v];
         R t0 = R(0), t1 = R(0), t2 = R(0);
         if (j < 2 && k < 2) {
-            const int* bt = nw.base_t + 3 * v;
-            const R* Wt = nw.W_t + 6 * v;
-            const int yj = node_at(bt[1], j, gd.n[1], gd.per[1]);
-            const int zk = node_at(bt[2], k, gd.n[2], gd.per[2]);
+            const int f[3] = {stencil_first(P.x, R(1.0)), stencil_first(P.y, R(1.0)), stencil_first(P.z, R(1.0))};
+            const int yj = node_at(stencil_base(f[1], gd.n[1], gd.per[1]), j, gd.n[1], gd.per[1]);
+            const int zk = node_at(stencil_base(f[2], gd.n[2], gd.per[2]), k, gd.n[2], gd.per[2]);
             if (yj >= 0 && zk >= 0) {
-                const R wy = Wt[2 + j], wz = Wt[4 + k];
+                const R ty = dirac<R>(BL_KERNEL_TOPHAT, (R)(f[1] + j) - P.y);
+                const R tz = dirac<R>(BL_KERNEL_TOPHAT, (R)(f[2] + k) - P.z);
                 for (int i = 0; i < 2; ++i) {
-                    const int xi = node_at(bt[0], i, gd.n[0], gd.per[0]);
+                    const int xi = node_at(stencil_base(f[0], gd.n[0], gd.per[0]), i, gd.n[0], gd.per[0]);
                     if (xi < 0) continue;
-                    const R w = (Wt[i] * wy) * wz;
+                    const R w = (dirac<R>(BL_KERNEL_TOPHAT, (R)(f[0] + i) - P.x) * ty) * tz;
                     const Vel4<C> u = ut[((size_t)xi * gd.n[1] + yj) * gd.n[2] + zk];
                     t0 += w * (R)u.x;
                     t1 += w * (R)u.y;
@@ -1088,11 +1161,18 @@ __global__ void __launch_bounds__(256) k_interp(InterpArgs<R> a)
 // are one 16x16x4 matrix instruction in the vertex real: per lane four LDS
 // reads and two multiplies, where a lane per cell took 24 reads and 24
 // fused multiply-adds for them (LDS reads bounded it).
+// Bound by vector instructions where many tiles are touched (a tile of 25
+// entries leaves lanes idle while their weights are formed), by latency on
+// one cell.  400 800 vertices, FP32: 183 us with a lane per cell, 159 with
+// the matrix instructions, 115 with one root per axis, the weights moved
+// to their cells by conditional shifts and the keys ranked, not sorted.
 // One launch (k_spread) holds two kinds of workgroups:
 //   small: tiles with at most kSmallTile entries (the touched-tile list,
 //          skipping the others), one wave per tile, four independent waves
-//          per workgroup, keys sorted in registers, one running sum from g
-//          in vertex order;
+//          per workgroup, keys ranked against each other in LDS (up
+//          to 64 entries are loaded as listed and staged in the column of
+//          their rank, up to 128 put in order first), one running sum from
+//          g in vertex order;
 //   big:   the big-tile list, one workgroup of four waves per tile; each
 //          wave sorts a run of 64 keys in registers and the runs are merged
 //          by rank in LDS (a bitonic sort in LDS past 256 entries); wave w
@@ -1135,72 +1215,92 @@ __device__ __forceinline__ void wave_sync()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Weights of list entry `e` on the tile's cells (rows 0-11: axis-major, 4
-// cells per axis) and its force (rows 12-14), into registers.  The vertex's
-// weights are loaded whole (not indexed by the stencil offset) so that no
-// load waits for the base.  A near-wall vertex's kernel part carries the
-// force times w (w < 1), its top-hat part the force times 1 - w (w > 0),
-// the top hat's two weights per axis.
+// Both kinds in one launch: workgroups [0, n_small) take the small tiles,
+// the others the big ones.
 template <class R>
-__device__ __forceinline__ void entry_weights(const Grid& gd, int Sw, const int org[3], int e,
-                                              const int* __restrict__ base, const R* __restrict__ W,
-                                              const R* __restrict__ vforce, const NearView<R>& nw, R ev[15])
+struct SpreadArgs {
+    LatView lv;
+    Grid gd;
+    int kernel, Sw, n_small;
+    double h;
+    // the touched-tile list (null: every tile is looked at, in space order)
+    const int *active, *nactive, *big, *nbig;
+    int ntiles, small;
+    FastDiv dty, dtz;  // division by the tiles along y and z
+    int* count;
+    int cap;
+    const int* list;
+    const Vel4<R>* vp;  // the binning's position copies
+    const R* vforce;
+    NearView<R> nw;
+    void* Fout;  // force field in the storage's force type
+    int xcd;     // order of the small-tile workgroups over the XCDs (ibm_block)
+};
+
+// List entry `e` as loaded: the vertex's position copy and its force, two
+// loads, where the stored base and weights were 60 B (FP32) on four lines.
+// A near-wall vertex's kernel part carries the force times w (w < 1), its
+// top-hat part the force times 1 - w (w > 0).
+template <class R>
+struct Entry {
+    Vel4<R> P;
+    R F[3];
+    bool top;
+};
+
+template <class R>
+__device__ __forceinline__ Entry<R> load_entry(const SpreadArgs<R>& A, int e)
 {
-    using R2 = typename Vec2<R>::T;
+    Entry<R> E;
     const bool nr = (e & kNearKey) != 0;
     const long v = nr ? (long)((e & ~kNearKey) >> 1) : (long)e;
-    const bool top = nr && (e & 1);
-    R w[12];
-    const int* bv;
-    int sw;
-    if (top) {
-        const R2* W2 = (const R2*)(nw.W_t + 6 * v);
-        for (int k = 0; k < 3; ++k) {
-            const R2 p = W2[k];
-            w[4 * k] = p.x;
-            w[4 * k + 1] = p.y;
-            w[4 * k + 2] = R(0.0);
-            w[4 * k + 3] = R(0.0);
-        }
-        bv = nw.base_t + 3 * v;
-        sw = 2;
-    } else {
-        const R2* W2 = (const R2*)(W + 12 * v);
-#pragma unroll
-        for (int k = 0; k < 6; ++k) {
-            const R2 p = W2[k];
-            w[2 * k] = p.x;
-            w[2 * k + 1] = p.y;
-        }
-        bv = base + 3 * v;
-        sw = Sw;
+    E.top = nr && (e & 1);
+    E.P = A.vp[v];
+    for (int k = 0; k < 3; ++k) E.F[k] = A.vforce[3 * v + k];
+    if (nr) {
+        const R wb = A.nw.blend[v];
+        const bool scale = E.top ? wb > R(0) : wb < R(1);
+        const R s = E.top ? R(1.) - wb : wb;
+        if (scale)
+            for (int k = 0; k < 3; ++k) E.F[k] *= s;
     }
+    return E;
+}
+
+// Its weights on the tile's cells (rows 0-11: axis-major, 4 cells per axis)
+// and its force (rows 12-14).
+template <class R>
+__device__ __forceinline__ void entry_weights(const SpreadArgs<R>& A, const int org[3], const Entry<R>& E, R ev[15])
+{
+    const Grid& gd = A.gd;
+    const R x[3] = {E.P.x, E.P.y, E.P.z};
+    const R h = A.nw.on && E.top ? R(1.0) : (R)A.h;
 #pragma unroll
     for (int ax = 0; ax < 3; ++ax) {
-        const int b = bv[ax];
+        const int first = stencil_first(x[ax], h);
+        const int b = stencil_base(first, gd.n[ax], gd.per[ax]);
+        W4<R> w = axis_weights<R>(A.kernel, x[ax], first);
+        if (A.nw.on) {
+            const W4<R> t = axis_weights<R>(BL_KERNEL_TOPHAT, x[ax], first);
+            w = {E.top ? t.w0 : w.w0, E.top ? t.w1 : w.w1, E.top ? t.w2 : w.w2, E.top ? t.w3 : w.w3};
+        }
+        // the tile's first node past the stencil's; a stencil that wrapped
+        // starts beyond the tile, and (but in a box of less than 8 nodes)
+        // reaches it only past the face
+        int d = org[ax] - b;
+        if (gd.per[ax] && d < -3) d += gd.n[ax];
+        R o[4];
+        shifted<R>(w, d, o);
+        if (gd.per[ax] && gd.n[ax] < 8) {  // both ends of a wrapped stencil may lie in one tile
+            R u[4];
+            shifted<R>(w, max(min(d + gd.n[ax], 4), -3), u);
 #pragma unroll
-        for (int l = 0; l < 4; ++l) {
-            int d = org[ax] + l - b;
-            if (gd.per[ax] && d < 0) d += gd.n[ax];
-            const R* wa = w + 4 * ax;
-            const R x = d == 0 ? wa[0] : (d == 1 ? wa[1] : (d == 2 ? wa[2] : wa[3]));
-            ev[4 * ax + l] = (unsigned)d < (unsigned)sw ? x : R(0.0);
+            for (int l = 0; l < 4; ++l) o[l] = d + l < 0 ? (d + gd.n[ax] <= 3 ? u[l] : R(0)) : o[l];
         }
+#pragma unroll
+        for (int l = 0; l < 4; ++l) ev[4 * ax + l] = o[l];
     }
-    R F0 = vforce[3 * v], F1 = vforce[3 * v + 1], F2 = vforce[3 * v + 2];
-    if (nr) {
-        const R wb = nw.blend[v];
-        const bool scale = top ? wb > R(0) : wb < R(1);
-        const R s = top ? R(1.) - wb : wb;
-        if (scale) {
-            F0 *= s;
-            F1 *= s;
-            F2 *= s;
-        }
-    }
-    ev[12] = F0;
-    ev[13] = F1;
-    ev[14] = F2;
+    for (int k = 0; k < 3; ++k) ev[12 + k] = E.F[k];
 }
 
 // Adds entries [0, cnt) of a staged half (cnt <= kChunk; the rows are zero
@@ -1226,9 +1326,7 @@ __device__ __forceinline__ void chunk_sum(const R (*ew)[kChunkRow], int cnt, int
 // Adds the sorted entries [lo, hi) of a tile to acc, 64 at a time; key(e)
 // gives the e-th sorted entry.
 template <class R, class KeyOf>
-__device__ __forceinline__ void sum_entries(const Grid& gd, int Sw, const int org[3], int lo, int hi, KeyOf key,
-                                            const int* __restrict__ base, const R* __restrict__ W,
-                                            const R* __restrict__ vforce, const NearView<R>& nw,
+__device__ __forceinline__ void sum_entries(const SpreadArgs<R>& A, const int org[3], int lo, int hi, KeyOf key,
                                             R (*ew)[kChunkRow], int lane, typename TileSum<R>::V& acc)
 {
     for (int c0 = lo; c0 < hi; c0 += 64) {
@@ -1236,7 +1334,7 @@ __device__ __forceinline__ void sum_entries(const Grid& gd, int Sw, const int or
         R ev[15];
 #pragma unroll
         for (int r = 0; r < 15; ++r) ev[r] = R(0.0);
-        if (e < hi) entry_weights(gd, Sw, org, key(e), base, W, vforce, nw, ev);
+        if (e < hi) entry_weights<R>(A, org, load_entry<R>(A, key(e)), ev);
 #pragma unroll
         for (int half = 0; half < 2; ++half) {
             const int cnt = min(kChunk, hi - c0 - half * kChunk);
@@ -1251,12 +1349,13 @@ __device__ __forceinline__ void sum_entries(const Grid& gd, int Sw, const int or
     }
 }
 
-__device__ __forceinline__ void tile_origin(const Grid& gd, int t, int org[3])
+template <class R>
+__device__ __forceinline__ void tile_origin(const SpreadArgs<R>& A, int t, int org[3])
 {
-    const int tz = t % gd.nt[2], rr = t / gd.nt[2], ty = rr % gd.nt[1], tx = rr / gd.nt[1];
-    org[0] = tx * kTile;
-    org[1] = ty * kTile;
-    org[2] = tz * kTile;
+    const unsigned rr = fdiv((unsigned)t, A.dtz), tx = fdiv(rr, A.dty);
+    org[0] = (int)tx * kTile;
+    org[1] = (int)(rr - tx * (unsigned)A.gd.nt[1]) * kTile;
+    org[2] = (int)((unsigned)t - rr * (unsigned)A.gd.nt[2]) * kTile;
 }
 
 // The body force of a lane's column, the start of its sums.
@@ -1273,11 +1372,26 @@ __device__ __forceinline__ void store_tile(const LatView& lv, const Grid& gd, co
 {
     const int comp = (lane >> 2) & 3, z = org[2] + (lane & 3);
     if (comp == 3 || z >= gd.n[2]) return;
+    FT* out = Fout + comp * lv.stride;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
         const int x = org[0] + TileSum<R>::x(lane, r), y = org[1] + TileSum<R>::y(lane, r);
-        if (x < gd.n[0] && y < gd.n[1]) Fout[comp * lv.stride + ((long)x * gd.n[1] + y) * gd.n[2] + z] = (FT)acc[r];
+        if (x < gd.n[0] && y < gd.n[1]) out[(unsigned)((x * gd.n[1] + y) * gd.n[2] + z)] = (FT)acc[r];
     }
+}
+
+// How many of the n keys in LDS (padded to a multiple of 4 with keys that
+// are below none) are below `mine`: four keys a read, the same address in
+// every lane.
+__device__ __forceinline__ int rank_in(const int* k, int n, int mine)
+{
+    int r = 0;
+#pragma unroll 4
+    for (int e = 0; e < n; e += 4) {
+        const int4 q = *(const int4*)(k + e);
+        r += (q.x < mine ? 1 : 0) + (q.y < mine ? 1 : 0) + (q.z < mine ? 1 : 0) + (q.w < mine ? 1 : 0);
+    }
+    return r;
 }
 
 // ascending bitonic sort of one key per lane across the wave
@@ -1306,37 +1420,75 @@ __device__ __forceinline__ int rank_in_run(const int* r, int key)
 }
 
 template <class FT, class R>
-__device__ __forceinline__ void spread_small(int blk, int nb, R (*ew_all)[15][kChunkRow], const LatView& lv,
-                                             const Grid& gd, int Sw, const int* __restrict__ active,
-                                             const int* __restrict__ nactive, int* __restrict__ count, int cap,
-                                             const int* __restrict__ list, const int* __restrict__ base,
-                                             const R* __restrict__ W, const R* __restrict__ vforce,
-                                             const NearView<R>& nw, FT* __restrict__ Fout)
+__device__ __forceinline__ void spread_small(int blk, int nb, int* keys, R (*ew_all)[15][kChunkRow],
+                                             const SpreadArgs<R>& A)
 {
+    const Grid& gd = A.gd;
+    const int* __restrict__ active = A.active;
+    int* __restrict__ count = A.count;
+    const int* __restrict__ list = A.list;
+    const int cap = A.cap;
     const int wv = threadIdx.x >> 6;
     R(*ew)[kChunkRow] = ew_all[wv];
-    const int na = *nactive;
+    const int na = active ? *A.nactive : A.ntiles;
     const int lane = threadIdx.x & 63;
     const int stride = nb * kSpreadWaves;
     int a = blk * kSpreadWaves + wv;
-    int t = a < na ? active[a] : 0;
+    int t = a < na ? (active ? active[a] : a) : 0;
     while (a < na) {
         // the list's first slots are loaded with the count (not after it),
         // and the next tile's id while this one is summed
         const int raw = list[(long)t * cap + lane];
         const int n = count[t];
         const int a_next = a + stride;
-        const int t_next = a_next < na ? active[a_next] : 0;
+        const int t_next = a_next < na ? (active ? active[a_next] : a_next) : 0;
         // a big tile is its workgroup's; a count already cleared (0) is one
         // that workgroup has finished (a listed tile has at least one entry)
-        if (n > 0 && n <= kSmallTile) {
-            const int key = wave_sort(lane < n ? raw : 0x7fffffff, lane);
+        if (n > 64 && n <= A.small) {
+            // two entries a lane: ordered through LDS, then 64 at a time
+            const int raw1 = lane < n - 64 ? list[(long)t * cap + 64 + lane] : 0x7fffffff;
+            int* k = keys + wv * kSmallTile;
+            k[lane] = raw;
+            k[64 + lane] = raw1;
+            wave_sync();
+            const int r0 = rank_in(k, n, raw), r1 = rank_in(k, n, raw1);
+            wave_sync();
+            k[r0] = raw;
+            if (lane < n - 64) k[r1] = raw1;
+            wave_sync();
             int org[3];
-            tile_origin(gd, t, org);
-            const R g = column_start<R>(lv, lane);
+            tile_origin<R>(A, t, org);
+            const R g = column_start<R>(A.lv, lane);
             typename TileSum<R>::V acc = {g, g, g, g};
-            sum_entries<R>(gd, Sw, org, 0, n, [&](int) { return key; }, base, W, vforce, nw, ew, lane, acc);
-            store_tile<FT, R>(lv, gd, org, lane, acc, Fout);
+            sum_entries<R>(A, org, 0, n, [&](int e) { return k[e]; }, ew, lane, acc);
+            store_tile<FT, R>(A.lv, gd, org, lane, acc, (FT*)A.Fout);
+            if (lane == 0) count[t] = 0;
+        } else if (n > 0 && n <= 64) {
+            // lane e takes entry e as listed and stages it in the column of
+            // its rank, so the loads do not wait for an order
+            int org[3];
+            tile_origin<R>(A, t, org);
+            const R g = column_start<R>(A.lv, lane);
+            typename TileSum<R>::V acc = {g, g, g, g};
+            const bool live = lane < n;
+            Entry<R> E = load_entry<R>(A, live ? raw : 0);
+            int* k = keys + wv * kSmallTile;
+            k[lane] = live ? raw : 0x7fffffff;
+            wave_sync();
+            const int rank = rank_in(k, n, raw);
+            const int col = live ? rank : lane;
+            if (!live) E.F[0] = E.F[1] = E.F[2] = R(0);
+            R ev[15];
+            entry_weights<R>(A, org, E, ev);
+            for (int h0 = 0; h0 < n; h0 += kChunk) {
+                if ((col & ~(kChunk - 1)) == h0)
+#pragma unroll
+                    for (int r = 0; r < 15; ++r) ew[r][col & (kChunk - 1)] = ev[r];
+                wave_sync();
+                chunk_sum<R>(ew, min(kChunk, n - h0), lane, acc);
+                wave_sync();
+            }
+            store_tile<FT, R>(A.lv, gd, org, lane, acc, (FT*)A.Fout);
             if (lane == 0) count[t] = 0;
         }
         a = a_next;
@@ -1346,20 +1498,19 @@ __device__ __forceinline__ void spread_small(int blk, int nb, R (*ew_all)[15][kC
 
 template <class FT, class R>
 __device__ __forceinline__ void spread_big(int blk, int nb, int* keys, int* runs, R (*ew_all)[15][kChunkRow],
-                                           R (*part)[4][64], const LatView& lv, const Grid& gd, int Sw,
-                                           const int* __restrict__ big, const int* __restrict__ nbig,
-                                           int* __restrict__ count, int cap, const int* __restrict__ list,
-                                           const int* __restrict__ base, const R* __restrict__ W,
-                                           const R* __restrict__ vforce, const NearView<R>& nw,
-                                           FT* __restrict__ Fout)
+                                           R (*part)[4][64], const SpreadArgs<R>& A)
 {
+    const Grid& gd = A.gd;
+    int* __restrict__ count = A.count;
+    const int* __restrict__ list = A.list;
+    const int cap = A.cap;
     const int wv = threadIdx.x >> 6;
     R(*ew)[kChunkRow] = ew_all[wv];
-    const int nt = *nbig;
+    const int nt = *A.nbig;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     for (int a = blk; a < nt; a += nb) {
-        const int t = big[a];
+        const int t = A.big[a];
         const int n = min(count[t], cap);  // a longer list was cut at binning and reported there
         const long o = (long)t * cap;
         if (n <= 64 * kSpreadWaves) {
@@ -1398,60 +1549,39 @@ __device__ __forceinline__ void spread_big(int blk, int nb, int* keys, int* runs
         }
         __syncthreads();
         int org[3];
-        tile_origin(gd, t, org);
+        tile_origin<R>(A, t, org);
         // wave w sums the contiguous range [lo, hi) of the sorted entries
         const int q = (n + kSpreadWaves - 1) / kSpreadWaves;
         const int lo = min(n, wv * q), hi = min(n, lo + q);
         typename TileSum<R>::V acc = {R(0), R(0), R(0), R(0)};
-        sum_entries<R>(gd, Sw, org, lo, hi, [&](int k) { return keys[k]; }, base, W, vforce, nw, ew, lane, acc);
+        sum_entries<R>(A, org, lo, hi, [&](int k) { return keys[k]; }, ew, lane, acc);
 #pragma unroll
         for (int r = 0; r < 4; ++r) part[wv][r][lane] = acc[r];
         __syncthreads();
         if (wv == 0) {
-            const R g = column_start<R>(lv, lane);
+            const R g = column_start<R>(A.lv, lane);
             acc = {g, g, g, g};
 #pragma unroll
             for (int w = 0; w < kSpreadWaves; ++w)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) acc[r] += part[w][r][lane];
-            store_tile<FT, R>(lv, gd, org, lane, acc, Fout);
+            store_tile<FT, R>(A.lv, gd, org, lane, acc, (FT*)A.Fout);
             if (lane == 0) count[t] = 0;
         }
         __syncthreads();  // keys and partial sums are rewritten for the next tile
     }
 }
 
-// Both kinds in one launch: workgroups [0, n_small) take the small tiles,
-// the others the big ones.
-template <class R>
-struct SpreadArgs {
-    LatView lv;
-    Grid gd;
-    int Sw, n_small;
-    const int *active, *nactive, *big, *nbig;
-    int* count;
-    int cap;
-    const int *list, *base;
-    const R *W, *vforce;
-    NearView<R> nw;
-    void* Fout;  // force field in the storage's force type
-    int xcd;     // order of the small-tile workgroups over the XCDs (ibm_block)
-};
-
 template <class S, class R>
 __device__ __forceinline__ void spread_body(int bx, int nbx, const SpreadArgs<R>& A)
 {
     using FT = typename Pop<S>::F;
-    __shared__ int keys[kMaxList];
+    __shared__ __align__(16) int keys[kMaxList];
     __shared__ int runs[64 * kSpreadWaves];
     __shared__ R ew_all[kSpreadWaves][15][kChunkRow];
     __shared__ R part[kSpreadWaves][4][64];
-    if (bx < A.n_small)
-        spread_small<FT, R>((int)ibm_block(bx, A.n_small, A.xcd), A.n_small, ew_all, A.lv, A.gd, A.Sw, A.active,
-                            A.nactive, A.count, A.cap, A.list, A.base, A.W, A.vforce, A.nw, (FT*)A.Fout);
-    else
-        spread_big<FT, R>(bx - A.n_small, nbx - A.n_small, keys, runs, ew_all, part, A.lv, A.gd, A.Sw, A.big, A.nbig,
-                          A.count, A.cap, A.list, A.base, A.W, A.vforce, A.nw, (FT*)A.Fout);
+    if (bx < A.n_small) spread_small<FT, R>((int)ibm_block(bx, A.n_small, A.xcd), A.n_small, keys, ew_all, A);
+    else spread_big<FT, R>(bx - A.n_small, nbx - A.n_small, keys, runs, ew_all, part, A);
 }
 
 template <class S, class R>
@@ -1469,7 +1599,7 @@ template <class R>
 __global__ void __launch_bounds__(256) k_bin_elem(BinArgs<R> b, int n1, ElemArgs<R> e)
 {
     const int bx = blockIdx.x;
-    if (bx < n1) bin_body<R>(ibm_block(bx, n1, b.xcd), b);
+    if (bx < n1) bin_one<R>(ibm_block(bx, n1, b.xcd), b);
     else elem_body<R>(ibm_block(bx - n1, (int)gridDim.x - n1, e.xcd), e);
 }
 
@@ -1927,8 +2057,6 @@ NearView<R> near_view(bl_ibm g)
     nw.on = g->has_boundary && g->v_near ? 1 : 0;
     nw.near = g->v_near;
     nw.blend = (R*)g->v_blend;
-    nw.base_t = g->v_base_t;
-    nw.W_t = (R*)g->v_w_t;
     return nw;
 }
 
@@ -1939,8 +2067,6 @@ int alloc_near(bl_ibm g)
     const size_t nv = (size_t)std::max<long>(g->NV, 1);
     hipError_t e = hipMalloc(&g->v_near, nv);
     if (e == hipSuccess) e = hipMalloc(&g->v_blend, (size_t)g->vreal * nv);
-    if (e == hipSuccess) e = hipMalloc(&g->v_base_t, sizeof(int) * 3 * nv);
-    if (e == hipSuccess) e = hipMalloc(&g->v_w_t, (size_t)g->vreal * 6 * nv);
     if (e != hipSuccess) return fail(BL_ERR_HIP, std::string("near-wall buffers: ") + hipGetErrorString(e));
     return BL_OK;
 }
@@ -2044,6 +2170,17 @@ int prep_bin(bl_ibm g, hipStream_t s)
     return BL_OK;
 }
 
+// With more vertices than tiles, about half the tiles or more are touched.
+// The spreading's waves then walk all of them in space order, sixteen
+// workgroups after one another on an XCD (the touched-tile list's order is
+// the binning's arrival), and a wave takes tiles of up to 128 entries: of
+// the 171 x 70 x 101 suspension's, spreading | interpolation 50.2 -> 46.6
+// us, and fewer tiles queue on the big-tile list's counter (binning of the
+// 400-cell one 100 -> 88 us).  One cell touches a few hundred tiles, fewer
+// than there are CUs for: there four waves take a tile past 64 entries
+// (2 562 vertices: 11.6 us against 15.7).
+bool spread_dense(bl_ibm g) { return g->NV >= g->lat->ntiles; }
+
 template <class R>
 BinArgs<R> bin_args(bl_ibm g)
 {
@@ -2055,8 +2192,7 @@ BinArgs<R> bin_args(bl_ibm g)
     a.h = g->h;
     a.NV = g->NV;
     a.pos = (const R*)g->pos;
-    a.base = g->v_base;
-    a.W = (R*)g->v_w;
+    a.vp = (Vel4<R>*)g->v_pos0;
     a.count = g->tile_count;
     a.list = g->tile_list;
     a.cap = kTileCap;
@@ -2067,10 +2203,14 @@ BinArgs<R> bin_args(bl_ibm g)
     a.pairs = g->n_active + 5 + g->alt;
     a.big = g->active + (2L + g->alt) * L->ntiles;
     a.nbig = g->n_active + 8 + g->alt;
+    a.small = spread_dense(g) ? kSmallTile : kSparseTile;
     a.nw = near_view<R>(g);
     a.xcd = g->lp[BL_IBM_XCD];
     return a;
 }
+
+// workgroups of a binning with bb threads each, iter vertices per lane group
+int bin_blocks(bl_ibm g, int bb, int iter) { return (int)nblk(g->NV, bb / kBinLanes * iter); }
 
 // host state after a binning has been enqueued
 void binned(bl_ibm g)
@@ -2089,7 +2229,9 @@ int do_bin(bl_ibm g, hipStream_t s, hipEvent_t done = nullptr)
         with_vreal(g, [&](auto tag) {
             using R = decltype(tag);
             const int bb = g->lp[BL_IBM_BIN_BLOCK];
-            hipLaunchKernelGGL(k_bin<R>, dim3(nblk(g->NV, bb)), dim3(bb), 0, s, bin_args<R>(g));
+            if (g->NV >= kManyVertices && !g->has_boundary)
+                hipLaunchKernelGGL(k_bin_many<R>, dim3(bin_blocks(g, bb, kBinMany)), dim3(bb), 0, s, bin_args<R>(g));
+            else hipLaunchKernelGGL(k_bin<R>, dim3(bin_blocks(g, bb, 1)), dim3(bb), 0, s, bin_args<R>(g));
             return 0;
         });
     if (done) BL_HIP(hipEventRecord(done, s));
@@ -2154,9 +2296,10 @@ InterpArgs<R> interp_args(bl_ibm g, const ListReset& lr)
 {
     InterpArgs<R> a;
     a.gd = grid_of(g->lat);
+    a.kernel = g->kernel;
+    a.h = g->h;
     a.NV = g->NV;
-    a.base = g->v_base;
-    a.W = (const R*)g->v_w;
+    a.vp = (const Vel4<R>*)g->v_pos0;
     a.ut = g->ut;
     a.vel = (R*)g->vel;
     a.pos = (R*)g->pos;
@@ -2220,20 +2363,26 @@ SpreadArgs<R> spread_args(bl_ibm g, unsigned& blocks, int share = 1)
     SpreadArgs<R> a;
     a.lv = ibm_view(g);
     a.gd = grid_of(L);
+    a.kernel = g->kernel;
     a.Sw = g->S;
-    a.active = g->active + (long)g->alt * L->ntiles;
+    a.h = g->h;
+    const bool dense = spread_dense(g);
+    a.small = dense ? kSmallTile : kSparseTile;
+    a.dty = make_fastdiv((unsigned)L->nty);
+    a.dtz = make_fastdiv((unsigned)L->ntz);
+    a.active = dense ? nullptr : g->active + (long)g->alt * L->ntiles;
+    a.ntiles = (int)L->ntiles;
     a.nactive = g->n_active + g->alt;
     a.big = g->active + (2L + g->alt) * L->ntiles;
     a.nbig = g->n_active + 8 + g->alt;
     a.count = g->tile_count;
     a.cap = kTileCap;
     a.list = g->tile_list;
-    a.base = g->v_base;
-    a.W = (const R*)g->v_w;
+    a.vp = (const Vel4<R>*)g->v_pos0;
     a.vforce = (const R*)g->force;
     a.nw = near_view<R>(g);
     a.Fout = g->force_alt;
-    a.xcd = g->lp[BL_IBM_XCD];
+    a.xcd = g->lp[BL_IBM_XCD] == 0 && dense ? 4 : g->lp[BL_IBM_XCD];
     // about one small-tile wave per touched tile and one workgroup per big
     // tile: the touched tiles are at most every tile and, for membranes,
     // fewer than the vertices (by default a wave per vertex); big tiles
@@ -2582,7 +2731,7 @@ int step_layered_s(bl_ibm g)
     if (!g->prepped && (rc = prep_bin(g, s))) return rc;
     g->prepped = false;
     const int bb = g->lp[BL_IBM_BIN_BLOCK];  // both halves of the paired launch
-    const int nb = (int)nblk(g->NV, bb), ne = (int)nblk(g->NT + g->NP + g->NL, bb);
+    const int nb = bin_blocks(g, bb, 1), ne = (int)nblk(g->NT + g->NP + g->NL, bb);
     hipLaunchKernelGGL(k_bin_elem<R>, dim3(nb + ne), dim3(bb), 0, s, bin_args<R>(g), nb, elem_args<R>(g));
     binned(g);
     const int gl = g->lp[BL_IBM_GATHER_LANES];
@@ -2688,7 +2837,7 @@ int plan_layered(bl_ibm g, LayeredEntry<R>& E, int share)
     g->prepped = false;
     E.bin = bin_args<R>(g);
     E.elem = elem_args<R>(g);
-    E.nb = (int)nblk(g->NV);
+    E.nb = bin_blocks(g, 256, 1);
     E.ne = (int)nblk(g->NT + g->NP + g->NL);
     binned(g);
     E.gather = gather_args<R>(g, true);
@@ -2724,7 +2873,7 @@ __global__ void __launch_bounds__(256) k_bin_elem_batch(const LayeredEntry<R>* _
     const int box = batch_box(base, nbox, (int)blockIdx.x);
     const LayeredEntry<R>& E = tab[box];
     const int bx = (int)blockIdx.x - base[box];
-    if (bx < E.nb) bin_body<R>(ibm_block(bx, E.nb, E.bin.xcd), E.bin);
+    if (bx < E.nb) bin_one<R>(ibm_block(bx, E.nb, E.bin.xcd), E.bin);
     else elem_body<R>(ibm_block(bx - E.nb, E.ne, E.elem.xcd), E.elem);
 }
 
@@ -3162,10 +3311,10 @@ int bl_ibm_destroy(bl_ibm g)
                     g->s_tri_area0, g->s_tri_geo0, g->s_rest, g->s_link, g->s_link_len, g->s_pair, g->s_pair_cs0,
                     g->s_vt_head, g->s_vt, g->s_vl_head, g->s_vl, g->s_vp_head, g->s_vp, g->s_area0, g->p_shape,
                     g->p_model, g->p_bug, g->p_params, g->p_voff, g->p_toff, g->p_loff, g->p_poff, g->p_geom,
-                    g->p_delta, g->pos, g->vel, g->force, g->ec, g->ut, g->v_base, g->v_w,
+                    g->p_delta, g->pos, g->vel, g->force, g->ec, g->ut, g->v_pos0,
                     g->tile_count, g->tile_list, g->active, g->n_active,
                     g->col_count, g->col_off, g->col_fill, g->col_z, g->n_hits, g->phase,
-                    g->flags_alt, g->force_alt, g->ch_part, g->ch_idx, g->p_choff, g->ch_partial, g->ch_tab, g->t_vert, g->v_inc, g->v_near, g->v_blend, g->v_base_t, g->v_w_t, g->v_part, g->t_part, g->r_part,
+                    g->flags_alt, g->force_alt, g->ch_part, g->ch_idx, g->p_choff, g->ch_partial, g->ch_tab, g->t_vert, g->v_inc, g->v_near, g->v_blend, g->v_part, g->t_part, g->r_part,
                     g->l_part, g->ext_force, g->r_state};
     for (void* p : ptrs) hipFree(p);
     interactions_free(g);
@@ -3349,7 +3498,7 @@ int bl_ibm_init(bl_ibm g)
         (rc = alloc_bytes(g->pos, vr * 3 * g->NV)) || (rc = alloc_bytes(g->vel, vr * 3 * g->NV)) ||
         (rc = alloc_bytes(g->force, vr * 3 * g->NV)) || (rc = alloc(g->p_geom, 11 * (size_t)g->np)) ||
         (rc = alloc(g->p_delta, 3 * (size_t)g->np)) || (rc = alloc_bytes(g->ec, vr * nec)) ||
-        (rc = alloc(g->v_base, 3 * g->NV)) || (rc = alloc_bytes(g->v_w, vr * 12 * g->NV)))
+        (rc = alloc_bytes(g->v_pos0, vr * 4 * g->NV)))
         return rc;
     if ((rc = vreal_upload(g, g->pos, 0, pos.data(), (long)pos.size(), L->stream))) return rc;
     g->ec_pair = 9 * g->NT;

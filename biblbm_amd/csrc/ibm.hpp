@@ -94,8 +94,6 @@ struct bl_ibm_s {
     bl_boundary boundary{};
     unsigned char* v_near = nullptr;  // per vertex: nearer than half support + 1
     void* v_blend = nullptr;          // per vertex: distance - half support (vreal)
-    int* v_base_t = nullptr;          // per vertex: top-hat stencil base (3)
-    void* v_w_t = nullptr;            // per vertex: top-hat weights (2 per axis, vreal)
 
     // ---- rigid particles (BL_MODEL_RIGID, rigid.hip) ----
     int n_rigid = 0;
@@ -119,8 +117,7 @@ struct bl_ibm_s {
     long pp_ncell = 0;
 
     // ---- stencil / tiles ----
-    int* v_base = nullptr;    // 3 per vertex
-    void* v_w = nullptr;      // 12 per vertex (3 axes x up to 4 weights, vreal)
+    void* v_pos0 = nullptr;   // per vertex: its position at the last binning and 1, or zeros (4, vreal)
     int* tile_count = nullptr;  // entries per tile (cleared by the spreading that consumes them)
     int* tile_list = nullptr;   // per tile a fixed-capacity list of the vertices whose stencil touches it
     int* active = nullptr;      // two lists of touched tiles, one per force-flag buffer, then the two
