@@ -2947,7 +2947,7 @@ struct EnsembleBatch {
     };
     struct Step {
         bool swapped = false;  // the IBM stages' AA parity (before the collision)
-        Launch reset, bin_elem, gather_stage, spread_interp, interp, geom_partial, geom_final, collide, vwall, vwall_u;
+        Launch reset, bin_elem, gather_stage, spread_interp, interp, geom_partial, geom_final, collide, vwall;
         CollidePlan c0;        // template choices of the collide launch
         bool vw_swapped = false;
     } step[2];
@@ -3124,18 +3124,16 @@ int ensemble_batch_build(const std::vector<bl_lattice>& lats, const std::vector<
         }
         st.collide = put_launch(img, put(img, views.data(), views.size()), cnt);
         std::vector<VwallPlan> vw;
-        std::vector<int> vcnt, ucnt;
+        std::vector<int> vcnt;
         st.vw_swapped = (lats[0]->steps & 1) != 0;
         for (bl_lattice L : lats)
             if (L->has_vwall && L->mask) {
-                vw.push_back(VwallPlan{view_of(L), L->nwall, L->d_wall});
-                vcnt.push_back((int)((L->nwall + 255) / 256));
-                ucnt.push_back((int)((2 * L->nwall + 255) / 256));
+                vw.push_back(VwallPlan{view_of(L), L->nwall});
+                vcnt.push_back(vwall_blocks(L));
             }
         B->any_vwall = !vw.empty();
         const size_t vtab = put(img, vw.data(), vw.size());
         st.vwall = put_launch(img, vtab, vcnt);
-        st.vwall_u = put_launch(img, vtab, ucnt);
     }
     for (size_t k = 0; k < n; ++k) lats[k]->steps = s0[k];
     if (rc) {  // a clear was due mid-step: the ensemble uses per-box branches
@@ -3172,8 +3170,7 @@ int ensemble_batch_launch(const EnsembleBatch* B, hipStream_t s)
         if (rc) return rc;
         if (st.vwall.nblk &&
             (rc = vwall_batch_launch(B->storage, st.vw_swapped, (const VwallPlan*)(d + st.vwall.tab),
-                                     (const int*)(d + st.vwall.base), (const int*)(d + st.vwall_u.base),
-                                     st.vwall.nbox, st.vwall.nblk, st.vwall_u.nblk, s)))
+                                     (const int*)(d + st.vwall.base), st.vwall.nbox, st.vwall.nblk, s)))
             return rc;
         if (B->fused) {
             ibm(true);

@@ -643,32 +643,31 @@ int collide_batch_launch(const CollidePlan& p0, bool emit, const LatView* views,
 // (PlaneFdBoundaryFunctional3D::processCell,
 // src/boundaryCondition/finiteDifferenceBoundaryProcessor3D.hh:68-115) with
 // the density rule of VelocityDirichletBoundaryDynamics::computeRhoBar
-// (src/boundaryCondition/boundaryDynamics.hh:631-660).  Two launches: the
-// first computes, from the post-stream state, the velocities that the
-// finite differences read (wall cells and the interior cells next to
-// them); the second rewrites every wall cell from its own post-stream
-// populations and those velocities.  A cell's population slots are its
-// own in either AA layout, so no wall cell reads a value another replaced.
-template <class S>
-__device__ void cell_velocity_post(const LatView& v, long c, int x, int y, int z, bool swapped, double u[3])
+// (src/boundaryCondition/boundaryDynamics.hh:631-660).  One launch rewrites
+// every wall cell from its own post-stream populations and the velocities
+// the finite differences read: of the interior cell next to it, and of its
+// four tangential neighbours, which on a wall plane are velocity-wall cells
+// themselves, so their velocity is the wall's and no population is loaded
+// (another kind of cell there has its velocity formed from its own slots).
+// A cell's population slots are its own in either AA layout and only
+// velocity-wall cells are written, so no wall cell reads a value another
+// replaced.
+// Bound by latency: a box's walls are a few thousand cells, two dependent
+// loads deep.  As a launch for the velocities (through a buffer) and one
+// for the cells, 256 lanes a workgroup and the axis a run-time index, the
+// 64^3 box's walls took 5.7 + 8.9 us; this takes 5.3 (even) and 8.1 (odd,
+// whose populations are the neighbours' slots); 64 boxes' 71 -> 40 us.
+constexpr int kVwallBlock = 64;  // a workgroup a wave: few cells spread over many CUs
+
+template <class S, bool SWAPPED>
+__device__ __forceinline__ void post_velocity(const LatView& v, long c, int x, int y, int z, double u[3])
 {
     using C = typename Pop<S>::C;
     using FT = typename Pop<S>::F;
-    const unsigned char m = v.mask ? v.mask[c] : (unsigned char)M_FLUID;
-    if (m == M_VWALL) {
-        const int p[3] = {x, y, z};
-        const int side = p[v.wall_axis] == 0 ? 0 : 1;
-        for (int d = 0; d < 3; ++d) u[d] = v.wall_u[3 * side + d];
-        return;
-    }
-    if (m == M_BB || m == M_NONE) {
-        u[0] = u[1] = u[2] = 0.0;
-        return;
-    }
     Nbr n;
-    n.init(v, x, y, z);
+    if (SWAPPED) n.init(v, x, y, z);
     C f[Q];
-    load_post<S>(v, n, c, swapped, f);
+    load_post<S>(v, n, c, SWAPPED, f);
     C F[3];
     cell_force<FT, C>(v, c, x, y, z, F);
     const C rb = sum_rho(f);
@@ -678,119 +677,114 @@ __device__ void cell_velocity_post(const LatView& v, long c, int x, int y, int z
     for (int d = 0; d < 3; ++d) u[d] = (double)(j[d] * invRho + F[d] / C(2));
 }
 
-__device__ __forceinline__ void wall_cell_coords(const LatView& v, long w, int& x, int& y, int& z)
-{
-    const int a = v.wall_axis;
-    const int n[3] = {v.nx, v.ny, v.nz};
-    const int t1 = a == 0 ? 1 : 0, t2 = a == 2 ? 1 : 2;
-    const long per_plane = (long)n[t1] * n[t2];
-    const int side = (int)(w / per_plane);
-    const long r = w % per_plane;
-    int p[3];
-    p[a] = side == 0 ? 0 : n[a] - 1;
-    p[t1] = (int)(r / n[t2]);
-    p[t2] = (int)(r % n[t2]);
-    x = p[0]; y = p[1]; z = p[2];
-}
-
-// Wall-plane index of a cell on plane `side` of the wall axis.
-__device__ __forceinline__ long wall_index(const LatView& v, int side, const int p[3])
-{
-    const int a = v.wall_axis;
-    const int n[3] = {v.nx, v.ny, v.nz};
-    const int t1 = a == 0 ? 1 : 0, t2 = a == 2 ? 1 : 2;
-    return (long)side * n[t1] * n[t2] + (long)p[t1] * n[t2] + p[t2];
-}
-
-// The velocities the finite differences of the wall cells read, computed
-// once per cell: cells w < nwall are the wall-plane cells themselves
-// (tangential neighbours), cells nwall + w the first interior cell next to
-// wall cell w (normal neighbour).  Three per cell in `out`.
-template <class S>
-__device__ __forceinline__ void vwall_u_cell(const LatView& v, long nwall, bool swapped, double* out, long w)
-{
-    if (w >= 2 * nwall) return;
-    const bool inner = w >= nwall;
-    int x, y, z;
-    wall_cell_coords(v, inner ? w - nwall : w, x, y, z);
-    if (inner) {
-        int q[3] = {x, y, z};
-        const int a = v.wall_axis;
-        q[a] += q[a] == 0 ? 1 : -1;
-        x = q[0];
-        y = q[1];
-        z = q[2];
-    }
-    double u[3];
-    cell_velocity_post<S>(v, ((long)x * v.ny + y) * v.nz + z, x, y, z, swapped, u);
-    double* o = out + 3 * w;
-    o[0] = u[0];
-    o[1] = u[1];
-    o[2] = u[2];
-}
-
-template <class S>
-__global__ void k_vwall_u(LatView v, long nwall, bool swapped, double* out)
-{
-    vwall_u_cell<S>(v, nwall, swapped, out, (long)blockIdx.x * blockDim.x + threadIdx.x);
-}
-
-template <class S>
-__device__ __forceinline__ void vwall_compute_cell(const LatView& v, long nwall, bool swapped, const double* un,
-                                                   long w)
+// Wall axis A; wall cell w counts plane 0, then plane n - 1, the later of
+// the two other axes fastest.
+template <class S, bool SWAPPED, int A>
+__device__ __forceinline__ void vwall_cell(const LatView& v, long nwall, long w)
 {
     using C = typename Pop<S>::C;
     using FT = typename Pop<S>::F;
+    constexpr int T1 = A == 0 ? 1 : 0, T2 = A == 2 ? 1 : 2;
     if (w >= nwall) return;
-    int x, y, z;
-    wall_cell_coords(v, w, x, y, z);
-    const long c = ((long)x * v.ny + y) * v.nz + z;
-    if (!v.mask || v.mask[c] != M_VWALL) return;
-    const int a = v.wall_axis;
-    const int p[3] = {x, y, z};
-    const int side = p[a] == 0 ? 0 : 1;
+    const int n3[3] = {v.nx, v.ny, v.nz};
+    const unsigned plane = (unsigned)n3[T1] * (unsigned)n3[T2], sd = (unsigned)w / plane;
+    const int side = sd ? 1 : 0;
+    const unsigned r = (unsigned)w - sd * plane;
+    int p[3];
+    p[A] = side == 0 ? 0 : n3[A] - 1;
+    p[T1] = (int)(r / (unsigned)n3[T2]);
+    p[T2] = (int)(r - (unsigned)p[T1] * (unsigned)n3[T2]);
+    const long c = ((long)p[0] * v.ny + p[1]) * v.nz + p[2];
     const int orient = side == 0 ? -1 : 1;
-    const double* uw = v.wall_u + 3 * side;
+    // the neighbours: 0 the interior cell, 1 / 2 the tangential ones of T1,
+    // 3 / 4 of T2
+    auto neighbour = [&](int k, int q[3]) {
+        q[0] = p[0];
+        q[1] = p[1];
+        q[2] = p[2];
+        if (k == 0) {
+            q[A] = min(max(p[A] + (side == 0 ? 1 : -1), 0), n3[A] - 1);
+            return ((long)q[0] * v.ny + q[1]) * v.nz + q[2];
+        }
+        auto step = [&](int t, int n, int per) {
+            return per ? (t < 0 ? t + n : (t >= n ? t - n : t)) : min(max(t, 0), n - 1);
+        };
+        const int s = k & 1 ? 1 : -1;
+        if (k <= 2) q[T1] = step(p[T1] + s, n3[T1], v.per[T1]);
+        else q[T2] = step(p[T2] + s, n3[T2], v.per[T2]);
+        return ((long)q[0] * v.ny + q[1]) * v.nz + q[2];
+    };
+    const unsigned char m = v.mask[c];
+    unsigned char mq[5];
+#pragma unroll
+    for (int k = 0; k < 5; ++k) {
+        int q[3];
+        mq[k] = v.mask[neighbour(k, q)];
+    }
+    if (m != M_VWALL) return;
+    const double uw[3] = {side ? v.wall_u[3] : v.wall_u[0], side ? v.wall_u[4] : v.wall_u[1],
+                          side ? v.wall_u[5] : v.wall_u[2]};
 
     Nbr n;
-    n.init(v, x, y, z);
+    if (SWAPPED) n.init(v, p[0], p[1], p[2]);
     C fc[Q];
-    load_post<S>(v, n, c, swapped, fc);
+    load_post<S>(v, n, c, SWAPPED, fc);
     C Fc[3];
-    cell_force<FT, C>(v, c, x, y, z, Fc);
-    double onWall = 0.0, normal = 0.0;
-    #pragma unroll
-    for (int i = 0; i < Q; ++i)
-        if (ci(i, a) == 0) onWall += (double)fc[i];
-    #pragma unroll
-    for (int i = 0; i < Q; ++i)
-        if (ci(i, a) == orient) normal += (double)fc[i];
-    const double velNormal = (double)orient * (uw[a] - 0.5 * (double)Fc[a]);
-    const double rb = (2.0 * normal + onWall - 1.0 * velNormal) / (1.0 + velNormal);
-    const double rho = rb + 1.0;
-
+    cell_force<FT, C>(v, c, p[0], p[1], p[2], Fc);
+    // the velocity of a neighbour: the wall's (of the plane it lies on) on a
+    // velocity-wall cell, zero on bounce-back and no-dynamics cells
+    auto velocity = [&](unsigned char mk, int k, double u[3]) {
+        int q[3];
+        const long cq = neighbour(k, q);
+        u[0] = u[1] = u[2] = 0.0;
+        if (mk == M_VWALL) {
+            const bool hi = q[A] != 0;
+            u[0] = hi ? v.wall_u[3] : v.wall_u[0];
+            u[1] = hi ? v.wall_u[4] : v.wall_u[1];
+            u[2] = hi ? v.wall_u[5] : v.wall_u[2];
+        } else if (mk == M_FLUID) {
+            post_velocity<S, SWAPPED>(v, cq, q[0], q[1], q[2], u);
+        }
+    };
     double du[3][3];
-    const int n3[3] = {v.nx, v.ny, v.nz};
-    for (int d = 0; d < 3; ++d) {
-        if (d == a) {
-            const double* u1 = un + 3 * (nwall + w);
-            for (int k = 0; k < 3; ++k) du[d][k] = -orient * (-uw[k] + u1[k]);
-        } else {
-            int qp[3] = {x, y, z}, qm[3] = {x, y, z};
-            qp[d] += 1;
-            qm[d] -= 1;
-            if (v.per[d]) {
-                if (qp[d] >= n3[d]) qp[d] -= n3[d];
-                if (qm[d] < 0) qm[d] += n3[d];
-            } else {
-                if (qp[d] >= n3[d]) qp[d] = n3[d] - 1;
-                if (qm[d] < 0) qm[d] = 0;
+    {
+        double u1[3];
+        velocity(mq[0], 0, u1);
+        for (int k = 0; k < 3; ++k) du[A][k] = -orient * (-uw[k] + u1[k]);
+    }
+    for (int k = 0; k < 3; ++k) du[T1][k] = du[T2][k] = 0.0;
+    if (!(mq[1] == M_VWALL && mq[2] == M_VWALL && mq[3] == M_VWALL && mq[4] == M_VWALL)) {
+        double d1[3] = {0.0, 0.0, 0.0}, d2[3] = {0.0, 0.0, 0.0};
+#pragma unroll 1
+        for (int t = 1; t < 5; ++t) {
+            double u[3];
+            velocity(t == 1 ? mq[1] : (t == 2 ? mq[2] : (t == 3 ? mq[3] : mq[4])), t, u);
+            for (int k = 0; k < 3; ++k) {
+                if (t == 1) d1[k] = u[k];
+                else if (t == 2) d1[k] -= u[k];
+                else if (t == 3) d2[k] = u[k];
+                else d2[k] -= u[k];
             }
-            const double* up = un + 3 * wall_index(v, side, qp);
-            const double* um = un + 3 * wall_index(v, side, qm);
-            for (int k = 0; k < 3; ++k) du[d][k] = (up[k] - um[k]) / 2.0;
+        }
+        for (int k = 0; k < 3; ++k) {
+            du[T1][k] = d1[k] / 2.0;
+            du[T2][k] = d2[k] / 2.0;
         }
     }
+    double onWall = 0.0, normal = 0.0;
+#pragma unroll
+    for (int i = 0; i < Q; ++i)
+        if (ci(i, A) == 0) onWall += (double)fc[i];
+    double lo = 0.0, hi = 0.0;
+#pragma unroll
+    for (int i = 0; i < Q; ++i) {
+        if (ci(i, A) == -1) lo += (double)fc[i];
+        if (ci(i, A) == 1) hi += (double)fc[i];
+    }
+    normal = side == 0 ? lo : hi;
+    const double velNormal = (double)orient * (uw[A] - 0.5 * (double)Fc[A]);
+    const double rb = (2.0 * normal + onWall - 1.0 * velNormal) / (1.0 + velNormal);
+    const double rho = rb + 1.0;
     const double sToPi = -rho / 3.0 / v.om_base;
     double pi[6];
     pi[0] = 2.0 * du[0][0] * sToPi;
@@ -802,7 +796,7 @@ __device__ __forceinline__ void vwall_compute_cell(const LatView& v, long nwall,
     const double jv[3] = {rho * uw[0], rho * uw[1], rho * uw[2]};
     const double jSqr = jv[0] * jv[0] + jv[1] * jv[1] + jv[2] * jv[2];
     const double invRho = 1.0 / (rb + 1.0);
-    #pragma unroll
+#pragma unroll
     for (int i = 0; i < Q; ++i) {
         const double c_j = cx(i) * jv[0] + cy(i) * jv[1] + cz(i) * jv[2];
         const double feq = tw(i) * (rb + 3. * c_j + invRho * (4.5 * c_j * c_j - 1.5 * jSqr));
@@ -820,69 +814,68 @@ __device__ __forceinline__ void vwall_compute_cell(const LatView& v, long nwall,
         fneq *= tw(i) * 3.0 * 3.0 / 2.0;
         fc[i] = (C)(feq + fneq);
     }
-    store_post<S>(v, n, c, swapped, fc);
+    store_post<S>(v, n, c, SWAPPED, fc);
 }
 
-template <class S>
-__global__ void k_vwall_compute(LatView v, long nwall, bool swapped, const double* un)
+template <class S, bool SWAPPED>
+__device__ __forceinline__ void vwall_body(const LatView& v, long nwall, long w)
 {
-    vwall_compute_cell<S>(v, nwall, swapped, un, (long)blockIdx.x * blockDim.x + threadIdx.x);
+    if (v.wall_axis == 0) vwall_cell<S, SWAPPED, 0>(v, nwall, w);
+    else if (v.wall_axis == 1) vwall_cell<S, SWAPPED, 1>(v, nwall, w);
+    else vwall_cell<S, SWAPPED, 2>(v, nwall, w);
 }
 
-// The velocity-wall passes of a batch of boxes (each with velocity walls
-// and no Guo wall): the same two launches, each over every box's wall
-// cells.
-// PHASE 0 neighbour velocities (base counts the workgroups over 2 nwall
-// cells), 1 the wall cells.
-template <class S, int PHASE>
-__global__ void k_vwall_batch(const VwallPlan* __restrict__ tab, const int* __restrict__ base, int nbox, bool swapped)
+template <class S, bool SWAPPED>
+__global__ void __launch_bounds__(kVwallBlock) k_vwall(LatView v, long nwall)
+{
+    vwall_body<S, SWAPPED>(v, nwall, (long)blockIdx.x * kVwallBlock + threadIdx.x);
+}
+
+// The velocity-wall pass of a batch of boxes (each with velocity walls and
+// no Guo wall): one launch over every box's wall cells.
+template <class S, bool SWAPPED>
+__global__ void __launch_bounds__(kVwallBlock) k_vwall_batch(const VwallPlan* __restrict__ tab,
+                                                             const int* __restrict__ base, int nbox)
 {
     const int box = batch_box(base, nbox, (int)blockIdx.x);
-    // the box's plan is read in place (a copy of it, which the wall
-    // velocity's indexed read would put in scratch memory, is not made)
-    const VwallPlan& w = tab[box];
-    const long i = (long)((int)blockIdx.x - base[box]) * blockDim.x + threadIdx.x;
-    if (PHASE == 0) vwall_u_cell<S>(w.v, w.nwall, swapped, w.buf, i);
-    else vwall_compute_cell<S>(w.v, w.nwall, swapped, w.buf, i);
+    const VwallPlan& w = tab[box];  // read in place
+    vwall_body<S, SWAPPED>(w.v, w.nwall, (long)((int)blockIdx.x - base[box]) * kVwallBlock + threadIdx.x);
 }
 
 template <class S>
-void vwall_batch_s(bool swapped, const VwallPlan* tab, const int* base, const int* base_u, int nbox, unsigned nblk,
-                   unsigned nblk_u, hipStream_t s)
+void vwall_batch_s(bool swapped, const VwallPlan* tab, const int* base, int nbox, unsigned nblk, hipStream_t s)
 {
-    hipLaunchKernelGGL((k_vwall_batch<S, 0>), dim3(nblk_u), dim3(256), 0, s, tab, base_u, nbox, swapped);
-    hipLaunchKernelGGL((k_vwall_batch<S, 1>), dim3(nblk), dim3(256), 0, s, tab, base, nbox, swapped);
+    if (swapped) hipLaunchKernelGGL((k_vwall_batch<S, true>), dim3(nblk), dim3(kVwallBlock), 0, s, tab, base, nbox);
+    else hipLaunchKernelGGL((k_vwall_batch<S, false>), dim3(nblk), dim3(kVwallBlock), 0, s, tab, base, nbox);
 }
 
-int vwall_batch_launch(int storage, bool swapped, const VwallPlan* tab, const int* base, const int* base_u, int nbox,
-                       unsigned nblk, unsigned nblk_u, hipStream_t s)
+int vwall_blocks(const bl_lattice_s* L) { return (int)((L->nwall + kVwallBlock - 1) / kVwallBlock); }
+
+int vwall_batch_launch(int storage, bool swapped, const VwallPlan* tab, const int* base, int nbox, unsigned nblk,
+                       hipStream_t s)
 {
-    if (storage == BL_STORE_F64) vwall_batch_s<double>(swapped, tab, base, base_u, nbox, nblk, nblk_u, s);
-    else if (storage == BL_STORE_F32) vwall_batch_s<float>(swapped, tab, base, base_u, nbox, nblk, nblk_u, s);
-    else vwall_batch_s<__half>(swapped, tab, base, base_u, nbox, nblk, nblk_u, s);
+    if (storage == BL_STORE_F64) vwall_batch_s<double>(swapped, tab, base, nbox, nblk, s);
+    else if (storage == BL_STORE_F32) vwall_batch_s<float>(swapped, tab, base, nbox, nblk, s);
+    else vwall_batch_s<__half>(swapped, tab, base, nbox, nblk, s);
     BL_CHECK_LAUNCH();
     return BL_OK;
+}
+
+template <class S>
+void vwall_s(const bl_lattice_s* L)
+{
+    const LatView v = view_of(L);
+    const dim3 nb((unsigned)vwall_blocks(L));
+    if (L->steps & 1) hipLaunchKernelGGL((k_vwall<S, true>), nb, dim3(kVwallBlock), 0, L->stream, v, L->nwall);
+    else hipLaunchKernelGGL((k_vwall<S, false>), nb, dim3(kVwallBlock), 0, L->stream, v, L->nwall);
 }
 
 int velocity_walls_launch(bl_lattice_s* L)
 {
     if (!L->has_vwall || !L->mask) return guo_walls_launch(L);
-    const LatView v = view_of(L);
-    const bool swapped = (L->steps & 1) != 0;
-    const unsigned nb = (unsigned)((L->nwall + 255) / 256), nbu = (unsigned)((2 * L->nwall + 255) / 256);
-    if (L->storage == BL_STORE_F64) {
-        hipLaunchKernelGGL(k_vwall_u<double>, dim3(nbu), dim3(256), 0, L->stream, v, L->nwall, swapped, L->d_wall);
-        hipLaunchKernelGGL(k_vwall_compute<double>, dim3(nb), dim3(256), 0, L->stream, v, L->nwall, swapped,
-                           (const double*)L->d_wall);
-    } else if (L->storage == BL_STORE_F32) {
-        hipLaunchKernelGGL(k_vwall_u<float>, dim3(nbu), dim3(256), 0, L->stream, v, L->nwall, swapped, L->d_wall);
-        hipLaunchKernelGGL(k_vwall_compute<float>, dim3(nb), dim3(256), 0, L->stream, v, L->nwall, swapped,
-                           (const double*)L->d_wall);
-    } else {
-        hipLaunchKernelGGL(k_vwall_u<__half>, dim3(nbu), dim3(256), 0, L->stream, v, L->nwall, swapped, L->d_wall);
-        hipLaunchKernelGGL(k_vwall_compute<__half>, dim3(nb), dim3(256), 0, L->stream, v, L->nwall, swapped,
-                           (const double*)L->d_wall);
-    }
+    if (L->storage == BL_STORE_F64) vwall_s<double>(L);
+    else if (L->storage == BL_STORE_F32) vwall_s<float>(L);
+    else vwall_s<__half>(L);
     BL_CHECK_LAUNCH();
     return guo_walls_launch(L);
 }
@@ -1289,7 +1282,6 @@ int bl_lattice_destroy(bl_lattice L)
     hipFree(L->tile_flags);
     hipFree(L->d_stage);
     hipFree(L->d_partials);
-    hipFree(L->d_wall);
     if (L->stream) hipStreamDestroy(L->stream);
     delete L;
     return BL_OK;
@@ -1368,14 +1360,7 @@ static int set_mask_cells(bl_lattice L, const unsigned char* mask)
                                                 "0 and n-1 of the wall axis (set it first)");
                 }
         const int t1 = a == 0 ? 1 : 0, t2 = a == 2 ? 1 : 2;
-        const long nwall = 2L * n[t1] * n[t2];
-        if (nwall > L->nwall) {
-            hipFree(L->d_wall);
-            // three neighbour velocities per wall cell and per interior
-            // cell next to it
-            BL_HIP(hipMalloc(&L->d_wall, sizeof(double) * 6 * nwall));
-        }
-        L->nwall = nwall;
+        L->nwall = 2L * n[t1] * n[t2];
     }
     return BL_OK;
 }

@@ -79,7 +79,6 @@ struct bl_lattice_s {
     // scratch
     double* d_stage = nullptr;  // ncell * 19 doubles, allocated on demand
     double* d_partials = nullptr;
-    double* d_wall = nullptr;   // velocities read by the velocity-wall finite differences
     long nwall = 0;
     bl_ibm ibm = nullptr;
     std::vector<bl_guo_wall> guo;  // inserted Guo curved walls (not owned)
@@ -148,17 +147,14 @@ bool collide_batchable(const CollidePlan& a, const CollidePlan& b);
 // level (0, 1, 2) of bl_lattice_set_launch_parity
 int collide_batch_launch(const CollidePlan& p0, bool emit, const LatView* views, const int* base, int nbox,
                          unsigned nblk, int order, int nt, hipStream_t s);
-// velocity-wall cells of one box: its view, wall-cell count and the buffer
-// of the velocities its finite differences read
+// velocity-wall cells of one box: its view and wall-cell count
 struct VwallPlan {
     LatView v;
     long nwall;
-    double* buf;
 };
-// base / nblk: workgroups over the wall cells, base_u / nblk_u over twice
-// as many (the neighbour-velocity pass)
-int vwall_batch_launch(int storage, bool swapped, const VwallPlan* tab, const int* base, const int* base_u, int nbox,
-                       unsigned nblk, unsigned nblk_u, hipStream_t s);
+int vwall_blocks(const bl_lattice_s* L);  // workgroups of its velocity-wall pass
+int vwall_batch_launch(int storage, bool swapped, const VwallPlan* tab, const int* base, int nbox, unsigned nblk,
+                       hipStream_t s);
 int ensure_force_field(bl_lattice_s* L);
 int collide_stream_launch(bl_lattice_s* L);
 int velocity_walls_launch(bl_lattice_s* L);  // post-stream passes: velocity walls, then Guo walls
