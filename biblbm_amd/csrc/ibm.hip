@@ -15,7 +15,7 @@
 //            deterministic, no float atomics);
 //   interp   U_k = sum phi phi phi u, one thread per vertex in the
 //            reference's node order (K4), fused with the advection x += U;
-//   move     per-particle area / volume / COM / bbox in FP64 with a
+//   move     per-particle area / volume / COM in FP64 with a
 //            fixed reduction order, COM mapped onto the periodic grid (K7);
 //   voxelize z-ray hits per column, sorted, parity fill of the phase (K8),
 //            only when the inner and outer viscosities differ.
@@ -36,6 +36,7 @@ namespace bl {
 
 namespace {
 
+constexpr int kGeomSums = 5;       // a particle's geometry: area, volume, centroid
 constexpr int kTileCap = 512;      // list entries per 4x4x4 tile (stencils touching it)
 constexpr int kSmallTile = 128;    // the most entries of a tile that one wave spreads (kSparseTile below)
 constexpr int kSparseTile = 64;    // the same where few tiles are touched: the others' waves are idle
@@ -743,7 +744,7 @@ __device__ void tri_forces(const ForceView<R>& f, int p, int s, int model, long 
         capsule_triangle<R>(v0, v1, v2, f.s_tri_geo0 + 4 * st, area0, P[0], P[1],
                             model != BL_MODEL_CAPSULE_NEOHOOKEAN, f.p_bug[p] != 0, -1, out);
     if (model == BL_MODEL_RBC || model == 3)
-        area_volume_triangle<R>(v0, v1, v2, area0, f.s_area0[s], f.p_geom[11 * p], f.p_geom[11 * p + 1], P[2], P[3],
+        area_volume_triangle<R>(v0, v1, v2, area0, f.s_area0[s], f.p_geom[kGeomSums * p], f.p_geom[kGeomSums * p + 1], P[2], P[3],
                                 P[4], P[5], out);
 }
 
@@ -1698,18 +1699,22 @@ __global__ void k_move(long NV, R* __restrict__ pos, const R* __restrict__ vel)
     pos[v] += vel[v];
 }
 
-// Per-particle area, signed volume, area-weighted centroid
-// (src/fsi/DeformableParticle3D.hh:54-82) and bounding box
-// (src/fsi/ParticleBase.hh:51-69) in FP64: each particle's triangles are cut
-// into chunks of 256 (one workgroup each, fixed-order tree in LDS), the
-// chunk partials are then summed in chunk order, so the result does not
-// depend on scheduling.
-// Chunk c (its row of `chunks`: first triangle, triangles, vertex range
-// of its bounding-box share, all global indices) -> 11 partials.
+// Per-particle area, signed volume and area-weighted centroid
+// (src/fsi/DeformableParticle3D.hh:54-82) in FP64, by a fixed reduction
+// order, so that the result does not depend on scheduling.  Every particle's
+// triangles are cut into chunks of 256 (one workgroup each, a tree in LDS)
+// and a second launch adds the chunk sums in chunk order; boundaries whose
+// particles all have at most kGeomTriangles triangles take one launch of a
+// workgroup per particle instead (k_geom: a lane's triangles one after the
+// other, a butterfly per wave, the waves in order).  Both wait for memory:
+// 1 280 triangles take 6.2 us in one launch, 4.5 + 4.6 in two, but 5 120
+// take 14 (each lane ten deep) against 9.1, and 400 cells of both sizes 22
+// against 16.
+constexpr long kGeomTriangles = 2048;
 template <class R>
 struct GeomArgs {
     ForceView<R> f;
-    const int4* chunks;
+    const int2* chunks;
     const int* t_vert;
     double* partial;
     int nchunk, np;
@@ -1722,124 +1727,143 @@ struct GeomArgs {
     const int* p_model;
 };
 
+// Adds one triangle's share to the sums.
+template <class R>
+__device__ __forceinline__ void triangle_sums(const R* pos, const int* tv, double acc[kGeomSums])
+{
+    const D3 v0 = ld3d(pos + 3 * (long)tv[0]), v1 = ld3d(pos + 3 * (long)tv[1]), v2 = ld3d(pos + 3 * (long)tv[2]);
+    const double dA = 0.5 * norm(cross(v1 - v0, v2 - v0));
+    acc[0] += dA;
+    acc[1] += dot(v0, cross(v1, v2)) / 6.;
+    acc[2] += ((v0.x + v1.x + v2.x) / 3.0) * dA;
+    acc[3] += ((v0.y + v1.y + v2.y) / 3.0) * dA;
+    acc[4] += ((v0.z + v1.z + v2.z) / 3.0) * dA;
+}
+
+// Chunk c (its row of `chunks`: first triangle, triangles, global indices)
+// -> its sums.
 template <class R>
 __device__ __forceinline__ void geom_partial_body(int c, const GeomArgs<R>& A)
 {
     const ForceView<R>& f = A.f;
-    const int4* __restrict__ chunks = A.chunks;
+    const int2* __restrict__ chunks = A.chunks;
     const int* __restrict__ t_vert = A.t_vert;
     double* __restrict__ partial = A.partial;
-    __shared__ double sh[11][256];
-    const int4 ch = chunks[c];
-    double acc[5] = {0, 0, 0, 0, 0};
-    if ((int)threadIdx.x < ch.y) {
-        const int* tv = t_vert + 3 * ((long)ch.x + threadIdx.x);
-        const D3 v0 = ld3d(f.pos + 3 * (long)tv[0]), v1 = ld3d(f.pos + 3 * (long)tv[1]),
-                 v2 = ld3d(f.pos + 3 * (long)tv[2]);
-        const double dA = 0.5 * norm(cross(v1 - v0, v2 - v0));
-        acc[0] = dA;
-        acc[1] = dot(v0, cross(v1, v2)) / 6.;
-        acc[2] = ((v0.x + v1.x + v2.x) / 3.0) * dA;
-        acc[3] = ((v0.y + v1.y + v2.y) / 3.0) * dA;
-        acc[4] = ((v0.z + v1.z + v2.z) / 3.0) * dA;
-    }
-    double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
-    for (long v = ch.z + threadIdx.x; v < ch.w; v += blockDim.x)
-        for (int d = 0; d < 3; ++d) {
-            const double x = (double)f.pos[3 * v + d];
-            lo[d] = fmin(lo[d], x);
-            hi[d] = fmax(hi[d], x);
-        }
-    for (int q = 0; q < 5; ++q) sh[q][threadIdx.x] = acc[q];
-    for (int d = 0; d < 3; ++d) {
-        sh[5 + 2 * d][threadIdx.x] = lo[d];
-        sh[6 + 2 * d][threadIdx.x] = hi[d];
-    }
+    __shared__ double sh[kGeomSums][256];
+    const int2 ch = chunks[c];
+    double acc[kGeomSums] = {0, 0, 0, 0, 0};
+    if ((int)threadIdx.x < ch.y) triangle_sums<R>(f.pos, t_vert + 3 * ((long)ch.x + threadIdx.x), acc);
+    for (int q = 0; q < kGeomSums; ++q) sh[q][threadIdx.x] = acc[q];
     __syncthreads();
     for (int w = 128; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) {
-            for (int q = 0; q < 5; ++q) sh[q][threadIdx.x] += sh[q][threadIdx.x + w];
-            for (int d = 0; d < 3; ++d) {
-                sh[5 + 2 * d][threadIdx.x] = fmin(sh[5 + 2 * d][threadIdx.x], sh[5 + 2 * d][threadIdx.x + w]);
-                sh[6 + 2 * d][threadIdx.x] = fmax(sh[6 + 2 * d][threadIdx.x], sh[6 + 2 * d][threadIdx.x + w]);
-            }
-        }
+        if ((int)threadIdx.x < w)
+            for (int q = 0; q < kGeomSums; ++q) sh[q][threadIdx.x] += sh[q][threadIdx.x + w];
         __syncthreads();
     }
-    if (threadIdx.x < 11) partial[11 * (long)c + threadIdx.x] = sh[threadIdx.x][0];
+    if (threadIdx.x < kGeomSums) partial[kGeomSums * (long)c + threadIdx.x] = sh[threadIdx.x][0];
 }
 
 template <class R>
 __global__ void __launch_bounds__(256) k_geom_partial(GeomArgs<R> a) { geom_partial_body<R>(blockIdx.x, a); }
 
-// Chunk partials -> geometry; the centre of mass is then mapped onto the
-// periodic grid (src/fsi/ParticleBase.hh:113-136, src/fsi/Periodicity.h:83-87)
-// and the whole particle shifted by the same amount.
+// A particle's sums -> geometry (one lane); the centre of mass is then
+// mapped onto the periodic grid (src/fsi/ParticleBase.hh:113-136,
+// src/fsi/Periodicity.h:83-87), `sft` the shift of the whole particle.
 template <class R>
-__device__ __forceinline__ void geom_final_body(int p, const GeomArgs<R>& A)
+__device__ __forceinline__ void geom_store(int p, const GeomArgs<R>& A, const double acc[kGeomSums], double sft[3])
 {
     const Grid& gd = A.gd;
-    const int* __restrict__ p_choff = A.p_choff;
-    const double* __restrict__ partial = A.partial;
-    const long* __restrict__ p_voff = A.p_voff;
-    double* __restrict__ geom = A.geom;
-    double* __restrict__ delta = A.delta;
-    R* __restrict__ pos = A.pos;
-    const int remap = A.remap;
-    const int* __restrict__ p_model = A.p_model;
-    __shared__ double sft[3];
-    __shared__ double part[64][11];  // a batch of chunk partials, loaded by all lanes at once
-    const int c0 = p_choff[p], c1 = p_choff[p + 1];
-    double acc[5] = {0, 0, 0, 0, 0};
-    double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
-    for (int b = c0; b < c1; b += 64) {
-        const int nb = min(64, c1 - b);
-        if ((int)threadIdx.x < nb)
-            for (int q = 0; q < 11; ++q) part[threadIdx.x][q] = partial[11 * (long)(b + threadIdx.x) + q];
-        __syncthreads();
-        if (threadIdx.x == 0)
-            for (int k = 0; k < nb; ++k) {  // chunk order
-                const double* P = part[k];
-                for (int q = 0; q < 5; ++q) acc[q] += P[q];
-                for (int d = 0; d < 3; ++d) {
-                    lo[d] = fmin(lo[d], P[5 + 2 * d]);
-                    hi[d] = fmax(hi[d], P[6 + 2 * d]);
-                }
-            }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        double* G = geom + 11 * p;
-        const double area = acc[0];
-        double com[3] = {acc[2] / area, acc[3] / area, acc[4] / area};
-        for (int d = 0; d < 3; ++d) {
-            sft[d] = 0.0;
-            // a rigid particle maps its own centre of mass (rigid.hip)
-            if (!remap || !gd.per[d] || p_model[p] == BL_MODEL_RIGID) continue;
+    double* G = A.geom + kGeomSums * p;
+    const double area = acc[0];
+    const double com[3] = {acc[2] / area, acc[3] / area, acc[4] / area};
+    G[0] = area;
+    G[1] = acc[1];
+    for (int d = 0; d < 3; ++d) {
+        sft[d] = 0.0;
+        G[2 + d] = com[d];
+        // a rigid particle maps its own centre of mass (rigid.hip)
+        if (A.remap && gd.per[d] && A.p_model[p] != BL_MODEL_RIGID) {
             const double L = (double)gd.n[d];
             const double x0 = -0.5;
             const double r = com[d] - L * floor((com[d] - x0) * (1. / L));
             sft[d] = r - com[d];
-            com[d] = r;
+            G[2 + d] = r;
         }
-        G[0] = area;
-        G[1] = acc[1];
-        for (int d = 0; d < 3; ++d) {
-            G[2 + d] = com[d];
-            G[5 + 2 * d] = lo[d] + sft[d];
-            G[6 + 2 * d] = hi[d] + sft[d];
-            delta[3 * p + d] = sft[d];
-        }
-    }
-    __syncthreads();
-    const double s0 = sft[0], s1 = sft[1], s2 = sft[2];
-    if (s0 == 0.0 && s1 == 0.0 && s2 == 0.0) return;
-    for (long v = p_voff[p] + threadIdx.x; v < p_voff[p + 1]; v += blockDim.x) {
-        pos[3 * v] = (R)((double)pos[3 * v] + s0);
-        pos[3 * v + 1] = (R)((double)pos[3 * v + 1] + s1);
-        pos[3 * v + 2] = (R)((double)pos[3 * v + 2] + s2);
+        A.delta[3 * p + d] = sft[d];
     }
 }
+
+// The shift of a whole particle by its workgroup.
+template <class R>
+__device__ __forceinline__ void geom_shift(int p, const GeomArgs<R>& A, const double sft[3])
+{
+    const double s0 = sft[0], s1 = sft[1], s2 = sft[2];
+    if (s0 == 0.0 && s1 == 0.0 && s2 == 0.0) return;
+    for (long v = A.p_voff[p] + threadIdx.x; v < A.p_voff[p + 1]; v += blockDim.x) {
+        A.pos[3 * v] = (R)((double)A.pos[3 * v] + s0);
+        A.pos[3 * v + 1] = (R)((double)A.pos[3 * v + 1] + s1);
+        A.pos[3 * v + 2] = (R)((double)A.pos[3 * v + 2] + s2);
+    }
+}
+
+// Chunk partials -> geometry.
+template <class R>
+__device__ __forceinline__ void geom_final_body(int p, const GeomArgs<R>& A)
+{
+    const int* __restrict__ p_choff = A.p_choff;
+    const double* __restrict__ partial = A.partial;
+    __shared__ double sft[3];
+    __shared__ double part[64][kGeomSums];  // a batch of chunk partials, loaded by all lanes at once
+    const int c0 = p_choff[p], c1 = p_choff[p + 1];
+    double acc[kGeomSums] = {0, 0, 0, 0, 0};
+    for (int b = c0; b < c1; b += 64) {
+        const int nb = min(64, c1 - b);
+        if ((int)threadIdx.x < nb)
+            for (int q = 0; q < kGeomSums; ++q)
+                part[threadIdx.x][q] = partial[kGeomSums * (long)(b + threadIdx.x) + q];
+        __syncthreads();
+        if (threadIdx.x == 0)
+            for (int k = 0; k < nb; ++k)  // chunk order
+                for (int q = 0; q < kGeomSums; ++q) acc[q] += part[k][q];
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) geom_store(p, A, acc, sft);
+    __syncthreads();
+    geom_shift(p, A, sft);
+}
+
+// One particle by one workgroup of kGeomBlock lanes: lane t takes triangles
+// t, t + kGeomBlock, ... in order, then a butterfly per wave and the waves
+// in order.
+constexpr int kGeomBlock = 512;
+
+template <class R>
+__device__ __forceinline__ void geom_body(int p, const GeomArgs<R>& A)
+{
+    __shared__ double wave[kGeomBlock / 64][kGeomSums];
+    __shared__ double sft[3];
+    const int tid = threadIdx.x;
+    double acc[kGeomSums] = {0, 0, 0, 0, 0};
+#pragma unroll 4
+    for (long t = A.f.p_toff[p] + tid; t < A.f.p_toff[p + 1]; t += kGeomBlock)
+        triangle_sums<R>(A.f.pos, A.t_vert + 3 * t, acc);
+    for (int o = 1; o < 64; o <<= 1)
+#pragma unroll
+        for (int q = 0; q < kGeomSums; ++q) acc[q] += __shfl_xor(acc[q], o);
+    if ((tid & 63) == 0)
+        for (int q = 0; q < kGeomSums; ++q) wave[tid >> 6][q] = acc[q];
+    __syncthreads();
+    if (tid == 0) {
+        for (int k = 1; k < kGeomBlock / 64; ++k)
+            for (int q = 0; q < kGeomSums; ++q) acc[q] += wave[k][q];
+        geom_store(p, A, acc, sft);
+    }
+    __syncthreads();
+    geom_shift(p, A, sft);
+}
+
+template <class R>
+__global__ void __launch_bounds__(kGeomBlock) k_geom(GeomArgs<R> a) { geom_body<R>(blockIdx.x, a); }
 
 template <class R>
 __global__ void __launch_bounds__(64) k_geom_final(GeomArgs<R> a) { geom_final_body<R>(blockIdx.x, a); }
@@ -2091,7 +2115,7 @@ GeomArgs<R> geom_args(bl_ibm g, int remap)
 {
     GeomArgs<R> a;
     a.f = force_view<R>(g);
-    a.chunks = (const int4*)g->ch_tab;
+    a.chunks = (const int2*)g->ch_tab;
     a.t_vert = g->t_vert;
     a.partial = g->ch_partial;
     a.nchunk = g->nchunk;
@@ -2113,6 +2137,10 @@ int update_particles(bl_ibm g, int remap, hipStream_t s)
     with_vreal(g, [&](auto tag) {
         using R = decltype(tag);
         const GeomArgs<R> a = geom_args<R>(g, remap);
+        if (g->geom_one) {
+            hipLaunchKernelGGL(k_geom<R>, dim3(g->np), dim3(kGeomBlock), 0, s, a);
+            return 0;
+        }
         hipLaunchKernelGGL(k_geom_partial<R>, dim3(g->nchunk), dim3(256), 0, s, a);
         hipLaunchKernelGGL(k_geom_final<R>, dim3(g->np), dim3(64), 0, s, a);
         return 0;
@@ -2926,6 +2954,14 @@ __global__ void __launch_bounds__(64) k_geom_final_batch(const LayeredEntry<R>* 
     geom_final_body<R>((int)blockIdx.x - base[box], tab[box].geom);
 }
 
+template <class R>
+__global__ void __launch_bounds__(kGeomBlock) k_geom_batch(const LayeredEntry<R>* __restrict__ tab,
+                                                           const int* __restrict__ base, int nbox)
+{
+    const int box = batch_box(base, nbox, (int)blockIdx.x);
+    geom_body<R>((int)blockIdx.x - base[box], tab[box].geom);
+}
+
 }  // namespace
 
 // Two coupled steps of every box of an ensemble as batched launches: the
@@ -2947,7 +2983,7 @@ struct EnsembleBatch {
     };
     struct Step {
         bool swapped = false;  // the IBM stages' AA parity (before the collision)
-        Launch reset, bin_elem, gather_stage, spread_interp, interp, geom_partial, geom_final, collide, vwall;
+        Launch reset, bin_elem, gather_stage, spread_interp, interp, geom_partial, geom_final, geom, collide, vwall;
         CollidePlan c0;        // template choices of the collide launch
         bool vw_swapped = false;
     } step[2];
@@ -2996,7 +3032,7 @@ int batch_plan_ibm(const std::vector<bl_ibm>& gs, std::vector<char>& img, Ensemb
         }
     }
     const size_t tab = put(img, E.data(), E.size());
-    std::vector<int> nr, nbe, ngs, nsi, nip, nch, npa;
+    std::vector<int> nr, nbe, ngs, nsi, nip, nch, npa, ngo;
     for (size_t k = 0; k < gs.size(); ++k) {
         nr.push_back(E[k].nr);
         nbe.push_back(E[k].nb + E[k].ne);
@@ -3005,8 +3041,9 @@ int batch_plan_ibm(const std::vector<bl_ibm>& gs, std::vector<char>& img, Ensemb
         ngs.push_back(E[k].ng + (fused ? 0 : E[k].nst));
         nsi.push_back(E[k].nsp + (fused ? 0 : E[k].nip));
         nip.push_back(fused ? E[k].nip : 0);
-        nch.push_back(gs[k]->nchunk);
-        npa.push_back(gs[k]->np);
+        nch.push_back(gs[k]->geom_one ? 0 : gs[k]->nchunk);
+        npa.push_back(gs[k]->geom_one ? 0 : gs[k]->np);
+        ngo.push_back(gs[k]->geom_one ? gs[k]->np : 0);
     }
     st.reset = put_launch(img, tab, nr);
     st.bin_elem = put_launch(img, tab, nbe);
@@ -3015,6 +3052,7 @@ int batch_plan_ibm(const std::vector<bl_ibm>& gs, std::vector<char>& img, Ensemb
     st.interp = put_launch(img, tab, nip);
     st.geom_partial = put_launch(img, tab, nch);
     st.geom_final = put_launch(img, tab, npa);
+    st.geom = put_launch(img, tab, ngo);
     return BL_OK;
 }
 
@@ -3055,6 +3093,7 @@ void batch_launch_ibm(const EnsembleBatch& B, const EnsembleBatch::Step& st, boo
     }
     go(k_geom_partial_batch<R>, st.geom_partial, 256);
     go(k_geom_final_batch<R>, st.geom_final, 64);
+    go(k_geom_batch<R>, st.geom, kGeomBlock);
 }
 
 }  // namespace
@@ -3311,7 +3350,7 @@ int bl_ibm_destroy(bl_ibm g)
                     g->p_delta, g->pos, g->vel, g->force, g->ec, g->ut, g->v_pos0,
                     g->tile_count, g->tile_list, g->active, g->n_active,
                     g->col_count, g->col_off, g->col_fill, g->col_z, g->n_hits, g->phase,
-                    g->flags_alt, g->force_alt, g->ch_part, g->ch_idx, g->p_choff, g->ch_partial, g->ch_tab, g->t_vert, g->v_inc, g->v_near, g->v_blend, g->v_part, g->t_part, g->r_part,
+                    g->flags_alt, g->force_alt, g->p_choff, g->ch_partial, g->ch_tab, g->t_vert, g->v_inc, g->v_near, g->v_blend, g->v_part, g->t_part, g->r_part,
                     g->l_part, g->ext_force, g->r_state};
     for (void* p : ptrs) hipFree(p);
     interactions_free(g);
@@ -3493,7 +3532,7 @@ int bl_ibm_init(bl_ibm g)
         (rc = upload(g->p_poff, poff)) || (rc = upload(g->p_shape, pshape)) || (rc = upload(g->p_model, pmodel)) ||
         (rc = upload(g->p_bug, pbug)) || (rc = upload(g->p_params, params)) ||
         (rc = alloc_bytes(g->pos, vr * 3 * g->NV)) || (rc = alloc_bytes(g->vel, vr * 3 * g->NV)) ||
-        (rc = alloc_bytes(g->force, vr * 3 * g->NV)) || (rc = alloc(g->p_geom, 11 * (size_t)g->np)) ||
+        (rc = alloc_bytes(g->force, vr * 3 * g->NV)) || (rc = alloc(g->p_geom, kGeomSums * (size_t)g->np)) ||
         (rc = alloc(g->p_delta, 3 * (size_t)g->np)) || (rc = alloc_bytes(g->ec, vr * nec)) ||
         (rc = alloc_bytes(g->v_pos0, vr * 4 * g->NV)))
         return rc;
@@ -3529,29 +3568,25 @@ int bl_ibm_init(bl_ibm g)
     BL_HIP(hipMalloc(&g->force_alt, 3 * L->stride * L->force_bytes));
     BL_HIP(hipMemset(g->force_alt, 0, 3 * L->stride * L->force_bytes));
     {
-        // chunks of 256 triangles per particle; chunk k also takes the
-        // bounding box of vertices [nv k / nch, nv (k + 1) / nch)
-        std::vector<int> chp, chi, choff{0}, tab, tvert;
+        // chunks of 256 triangles per particle
+        std::vector<int> choff{0}, tab, tvert;
         tvert.reserve(3 * (size_t)g->NT);
         for (int p = 0; p < g->np; ++p) {
             const ShapeHost& S = g->shapes[g->parts[p].shape];
-            const long nt = toff[p + 1] - toff[p], nv = voff[p + 1] - voff[p];
+            const long nt = toff[p + 1] - toff[p];
             const int nch = (int)std::max<long>(1, (nt + 255) / 256);
             for (int k = 0; k < nch; ++k) {
-                chp.push_back(p);
-                chi.push_back(k);
                 tab.push_back((int)(toff[p] + 256L * k));
                 tab.push_back((int)std::max<long>(0, std::min<long>(256, nt - 256L * k)));
-                tab.push_back((int)(voff[p] + nv * k / nch));
-                tab.push_back((int)(voff[p] + nv * (k + 1) / nch));
             }
             choff.push_back(choff.back() + nch);
             for (long t = 0; t < 3 * nt; ++t) tvert.push_back((int)(voff[p] + S.tri[t]));
         }
-        g->nchunk = (int)chp.size();
-        if ((rc = upload(g->ch_part, chp)) || (rc = upload(g->ch_idx, chi)) || (rc = upload(g->p_choff, choff)) ||
-            (rc = upload(g->ch_tab, tab)) || (rc = upload(g->t_vert, tvert)) ||
-            (rc = alloc(g->ch_partial, 11 * (size_t)std::max(g->nchunk, 1))))
+        g->nchunk = (int)tab.size() / 2;
+        g->geom_one = true;
+        for (int p = 0; p < g->np; ++p) g->geom_one = g->geom_one && toff[p + 1] - toff[p] <= kGeomTriangles;
+        if ((rc = upload(g->p_choff, choff)) || (rc = upload(g->ch_tab, tab)) || (rc = upload(g->t_vert, tvert)) ||
+            (rc = alloc(g->ch_partial, kGeomSums * (size_t)std::max(g->nchunk, 1))))
             return rc;
     }
     BL_HIP(hipMemset(g->tile_count, 0, L->ntiles * sizeof(int)));
@@ -3859,12 +3894,12 @@ int bl_rbc_shrink_volume(bl_ibm g, int pid, double vol_final, int n_it, double d
             if ((rc = update_particles(g, 0, s)) || (rc = membrane_forces(g, s))) return rc;
         }
         // a particle whose area went NaN starts over with twice the damping
-        std::vector<double> geom(11 * (size_t)np);
+        std::vector<double> geom(kGeomSums * (size_t)np);
         BL_HIP(hipMemcpyAsync(geom.data(), g->p_geom, sizeof(double) * geom.size(), hipMemcpyDeviceToHost, s));
         BL_HIP(hipStreamSynchronize(s));
         for (int p = 0; p < np; ++p) {
             if (!todo[p]) continue;
-            const double area = geom[11 * p];
+            const double area = geom[kGeomSums * p];
             if (area == area) {
                 todo[p] = 0;
                 continue;
@@ -3992,8 +4027,8 @@ int bl_particle_observables(bl_ibm g, int pid, double out[14])
     int rc = need_init(g);
     if (rc) return rc;
     if (!out || pid < 0 || pid >= g->np) return fail(BL_ERR_ARG, "bl_particle_observables: bad argument");
-    double geom[11];
-    BL_HIP(hipMemcpyAsync(geom, g->p_geom + 11 * pid, sizeof(geom), hipMemcpyDeviceToHost, g->lat->stream));
+    double geom[kGeomSums];
+    BL_HIP(hipMemcpyAsync(geom, g->p_geom + kGeomSums * pid, sizeof(geom), hipMemcpyDeviceToHost, g->lat->stream));
     const int nv = g->shapes[g->parts[pid].shape].nv;
     std::vector<double> pos(3 * (size_t)nv);
     rc = bl_particle_get(g, pid, 0, pos.data());

@@ -66,7 +66,7 @@ struct bl_ibm_s {
     long* p_toff = nullptr;
     long* p_loff = nullptr;
     long* p_poff = nullptr;
-    double* p_geom = nullptr;    // 11 per particle: area, volume, com(3), bbox(6)
+    double* p_geom = nullptr;    // 5 per particle: area, volume, com(3)
     double* p_delta = nullptr;   // 3 per particle (COM remap shift)
     int* v_part = nullptr;       // particle of each vertex, triangle, pair, link
     int* v_inc = nullptr;        // per vertex: incidence list starts and counts, particle (8 ints)
@@ -130,12 +130,11 @@ struct bl_ibm_s {
     bool alt_full = false;      // flags_alt has every tile set: the next binning clears all of it
     unsigned char* flags_alt = nullptr;  // next step's tile flags (swapped with the lattice's)
     void* force_alt = nullptr;           // next step's force field (swapped with the lattice's)
-    int* ch_part = nullptr;              // per geometry chunk: particle
-    int* ch_idx = nullptr;               //                     chunk index within the particle
     int* p_choff = nullptr;              // np+1 chunk offsets
     int nchunk = 0;
-    double* ch_partial = nullptr;        // 11 per chunk
-    int* ch_tab = nullptr;               // per chunk: first triangle, triangles, bbox vertex range (4)
+    bool geom_one = false;               // every particle small enough for a workgroup (k_geom)
+    double* ch_partial = nullptr;        // 5 per chunk
+    int* ch_tab = nullptr;               // per chunk: first triangle, triangles
     int* t_vert = nullptr;               // per triangle: its three global vertex indices
 
     // ---- voxelization ----
