@@ -1870,15 +1870,31 @@ __global__ void __launch_bounds__(64) k_geom_final(GeomArgs<R> a) { geom_final_b
 
 // --------------------------------------------------------- voxelization
 // z-rays through integer (x, y) columns (RayTracer::find_intersections_z,
-// src/fsi/RayTracer.hh:19-39,80-108).  Pass 0 counts hits per column,
-// pass 1 writes them (z mapped into [-0.5, nz - 0.5) on a periodic z axis,
-// as ZBuffer::put does, src/fsi/ZBuffer.h:39-49).
+// src/fsi/RayTracer.hh:19-39,80-108; z mapped into [-0.5, nz - 0.5) on a
+// periodic z axis, as ZBuffer::put does, src/fsi/ZBuffer.h:39-49), then the
+// fill of apply_voxelization (src/fsi/ImmersedBoundaryDynamics_voxelization.hh:
+// 121-165): between consecutive sorted hits the nodes alternate outside and
+// inside, a later segment overwriting a shared end node.  A node is
+// therefore inside when an odd number of hits lie at or below it, and the
+// hits of a column need neither a list nor an order: each toggles the bit of
+// the first node at or above it, and the fill takes the parity of the bits
+// up to a node.  Only the last node differs: the fill's tail runs where the
+// last hit's first node comes before it, so with that hit between the last
+// two nodes the last one keeps its value, and with a hit exactly on it it
+// takes the value before that hit; a flag word per column says so.
+// Bound by latency.  As hit counts, a scan, a second trace into lists and a
+// sort per column this was six launches and 44 us for 5 120 triangles on 75
+// x 61 columns of 83 nodes; two launches and 9.4 us.
+constexpr int kFillCols = 16;  // columns a workgroup fills
+constexpr unsigned kHitBeyond = 1, kHitOnLast = 2, kHitBeforeLast = 4;
+
+__host__ __device__ inline int column_words(int nz) { return (nz + 31) / 32 + 1; }
+
+// One triangle's hits into the columns' bits; returns their number.
 template <class R>
-__global__ void k_ray_hits(ForceView<R> f, Grid gd, long NT, int pass, int* col_count, const int* col_off,
-                           int* col_fill, double* col_z, long cap, int* status)
+__device__ __forceinline__ int trace_triangle(const ForceView<R>& f, const Grid& gd, long g, long NT, unsigned* bits)
 {
-    const long g = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= NT) return;
+    if (g >= NT) return 0;
     const int p = f.t_part[g];
     const int s = f.p_shape[p];
     const long vo = f.p_voff[p];
@@ -1888,16 +1904,18 @@ __global__ void k_ray_hits(ForceView<R> f, Grid gd, long NT, int pass, int* col_
     // a triangle with a non-finite corner, or wider than the lattice, is
     // not traced (its membrane diverged; the binning reports it)
     const double ext = fmax(fmax(fabs(a.x), fabs(b.x)), fmax(fmax(fabs(c.x), fabs(a.y)), fmax(fabs(b.y), fabs(c.y))));
-    if (!(ext < 1e9)) return;
+    if (!(ext < 1e9)) return 0;
     const long x0 = (long)ceil(fmin(a.x, fmin(b.x, c.x))), x1 = (long)floor(fmax(a.x, fmax(b.x, c.x)));
     const long y0 = (long)ceil(fmin(a.y, fmin(b.y, c.y))), y1 = (long)floor(fmax(a.y, fmax(b.y, c.y)));
-    if (x1 - x0 > (long)gd.n[0] + 4 || y1 - y0 > (long)gd.n[1] + 4) return;
+    if (x1 - x0 > (long)gd.n[0] + 4 || y1 - y0 > (long)gd.n[1] + 4) return 0;
     const D3 e1 = b - a, e2 = c - a;
     const D3 dir = {0, 0, 1};
     const D3 q = cross(dir, e2);
     const double det = dot(e1, q);
-    if (fabs(det) < 2.220446049250313e-16) return;
+    if (fabs(det) < 2.220446049250313e-16) return 0;
     const double fi = 1 / det;
+    const int W = column_words(gd.n[2]);
+    int hits = 0;
     for (long i = x0; i <= x1; ++i)
         for (long j = y0; j <= y1; ++j) {
             const D3 o = {(double)i, (double)j, 0.};
@@ -1911,81 +1929,68 @@ __global__ void k_ray_hits(ForceView<R> f, Grid gd, long NT, int pass, int* col_
             const int cy_ = wrap_node((int)j, gd.n[1], gd.per[1]);
             if (cx_ < 0 || cy_ < 0) continue;
             const long col = (long)cx_ * gd.n[1] + cy_;
-            if (pass == 0) {
-                atomicAdd(&col_count[col], 1);
-            } else {
-                double z = fi * dot(e2, r);
-                if (gd.per[2]) {
-                    const double L = (double)gd.n[2];
-                    z = z - L * floor((z + 0.5) * (1. / L));
-                }
-                const long slot = (long)col_off[col] + atomicAdd(&col_fill[col], 1);
-                if (slot < cap) col_z[slot] = z;
-                else atomicOr(&status[2], 2);
+            double z = fi * dot(e2, r);
+            if (gd.per[2]) {
+                const double L = (double)gd.n[2];
+                z = z - L * floor((z + 0.5) * (1. / L));
+            }
+            ++hits;
+            const int last = gd.n[2] - 1;
+            unsigned* b = bits + col * W;
+            if (z > (double)last) {
+                atomicOr(&b[W - 1], kHitBeyond);
+                continue;
+            }
+            const double node = fmax(ceil(z), 0.0);
+            const int k = (int)node;
+            atomicXor(&b[k >> 5], 1u << (k & 31));
+            if (ceil(z) == (double)last) atomicOr(&b[W - 1], z == (double)last ? kHitOnLast : kHitBeforeLast);
+        }
+    return hits;
+}
+
+template <class R>
+__global__ void __launch_bounds__(256) k_ray_hits(ForceView<R> f, Grid gd, long NT, unsigned* bits, int* total)
+{
+    __shared__ int hits;
+    if (threadIdx.x == 0) hits = 0;
+    __syncthreads();
+    const int n = trace_triangle<R>(f, gd, (long)blockIdx.x * blockDim.x + threadIdx.x, NT, bits);
+    if (n) atomicAdd(&hits, n);
+    __syncthreads();
+    if (threadIdx.x == 0 && hits) atomicAdd(total, hits);
+}
+// Fills kFillCols columns per workgroup, a lane per node (consecutive bytes),
+// and clears their bits for the next step.  `cap`: the most hits a step may
+// have.
+__global__ void __launch_bounds__(256) k_fill_columns(Grid gd, unsigned* bits, int* total, long cap, int* status,
+                                                      unsigned char* phase)
+{
+    const int nz = gd.n[2], W = column_words(nz);
+    const long ncol = (long)gd.n[0] * gd.n[1], c0 = (long)blockIdx.x * kFillCols;
+    const int nc = (int)(ncol - c0 < kFillCols ? ncol - c0 : kFillCols);
+    unsigned* b = bits + c0 * W;
+    for (int i = threadIdx.x; i < nc * nz; i += blockDim.x) {
+        const int col = (int)((unsigned)i / (unsigned)nz), z = i - col * nz;
+        const unsigned* w = b + col * W;
+        unsigned x = w[z >> 5] & (0xffffffffu >> (31 - (z & 31)));
+        for (int k = 0; k < (z >> 5); ++k) x ^= w[k];
+        unsigned char in = __popc(x) & 1;
+        if (z == nz - 1) {
+            const unsigned fl = w[W - 1];
+            if (!(fl & kHitBeyond)) {
+                if (fl & kHitOnLast) in ^= 1;
+                else if (fl & kHitBeforeLast) continue;
             }
         }
-}
-
-// Per column: sort the hits and fill the phase as apply_voxelization does
-// (src/fsi/ImmersedBoundaryDynamics_voxelization.hh:121-165): alternate
-// outside/inside between consecutive hits, later segments overwrite the
-// shared end node.
-__global__ void k_fill_columns(Grid gd, const int* col_count, const int* col_off, double* col_z, long cap,
-                               unsigned char* phase)
-{
-    const long col = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (col >= (long)gd.n[0] * gd.n[1]) return;
-    const int nz = gd.n[2];
-    unsigned char* ph = phase + col * nz;
-    int n = col_count[col];
-    const long o = col_off[col];
-    if (o + n > cap) n = (int)(cap > o ? cap - o : 0);
-    double* zs = col_z + o;
-    for (int i = 1; i < n; ++i) {  // insertion sort (few hits per column)
-        const double key = zs[i];
-        int j = i - 1;
-        while (j >= 0 && zs[j] > key) {
-            zs[j + 1] = zs[j];
-            --j;
-        }
-        zs[j + 1] = key;
+        phase[c0 * nz + i] = in;
     }
-    bool inside = false;
-    double z_last = -10000;
-    for (int k = 0; k < n; ++k) {
-        const long zlo = max((long)ceil(z_last), 0L), zhi = min((long)floor(zs[k]), (long)nz - 1);
-        for (long z = zlo; z <= zhi; ++z) ph[z] = inside ? 1 : 0;
-        z_last = zs[k];
-        inside = !inside;
+    __syncthreads();
+    for (int i = threadIdx.x; i < nc * W; i += blockDim.x) b[i] = 0;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        if (*total > cap) atomicOr(&status[2], 2);
+        *total = 0;
     }
-    if (ceil(z_last) < nz - 1) {
-        const long zlo = max((long)ceil(z_last), 0L);
-        for (long z = zlo; z <= nz - 1; ++z) ph[z] = inside ? 1 : 0;
-    }
-}
-
-__global__ void k_scan_cols(const int* in, long n, int* off, int* total)
-{
-    // single-workgroup exclusive scan (columns are few: nx*ny)
-    __shared__ int sh[256];
-    int carry = 0;
-    for (long c0 = 0; c0 < n; c0 += 256) {
-        const long i = c0 + threadIdx.x;
-        const int v = i < n ? in[i] : 0;
-        sh[threadIdx.x] = v;
-        __syncthreads();
-        for (int o = 1; o < 256; o <<= 1) {
-            const int t = (int)threadIdx.x >= o ? sh[threadIdx.x - o] : 0;
-            __syncthreads();
-            sh[threadIdx.x] += t;
-            __syncthreads();
-        }
-        if (i < n) off[i] = carry + sh[threadIdx.x] - v;
-        const int tot = sh[255];
-        __syncthreads();
-        carry += tot;
-    }
-    if (threadIdx.x == 0) *total = carry;
 }
 
 }  // namespace
@@ -2568,22 +2573,14 @@ int do_voxelize(bl_ibm g, hipStream_t s)
     bl_lattice L = g->lat;
     if (L->omega_c0 == L->omega_c1 || g->NT == 0) return BL_OK;
     const Grid gd = grid_of(L);
-    const long ncol = (long)L->nx * L->ny;
-    hipLaunchKernelGGL(k_fill_i32, dim3(nblk(ncol)), dim3(256), 0, s, g->col_count, ncol, 0);
-    hipLaunchKernelGGL(k_fill_i32, dim3(nblk(ncol)), dim3(256), 0, s, g->col_fill, ncol, 0);
     with_vreal(g, [&](auto tag) {
         using R = decltype(tag);
-        const ForceView<R> f = force_view<R>(g);
-        hipLaunchKernelGGL(k_ray_hits<R>, dim3(nblk(g->NT)), dim3(256), 0, s, f, gd, g->NT, 0, g->col_count,
-                           (const int*)g->col_off, g->col_fill, g->col_z, g->col_cap, g->n_active);
-        hipLaunchKernelGGL(k_scan_cols, dim3(1), dim3(256), 0, s, (const int*)g->col_count, ncol, g->col_off,
+        hipLaunchKernelGGL(k_ray_hits<R>, dim3(nblk(g->NT)), dim3(256), 0, s, force_view<R>(g), gd, g->NT, g->col_bits,
                            g->n_hits);
-        hipLaunchKernelGGL(k_ray_hits<R>, dim3(nblk(g->NT)), dim3(256), 0, s, f, gd, g->NT, 1, g->col_count,
-                           (const int*)g->col_off, g->col_fill, g->col_z, g->col_cap, g->n_active);
         return 0;
     });
-    hipLaunchKernelGGL(k_fill_columns, dim3(nblk(ncol)), dim3(256), 0, s, gd, (const int*)g->col_count,
-                       (const int*)g->col_off, g->col_z, g->col_cap, g->phase);
+    hipLaunchKernelGGL(k_fill_columns, dim3(nblk((long)L->nx * L->ny, kFillCols)), dim3(256), 0, s, gd, g->col_bits,
+                       g->n_hits, g->hit_cap, g->n_active, g->phase);
     BL_CHECK_LAUNCH();
     if (L->phase != g->phase) {
         L->phase = g->phase;
@@ -3349,7 +3346,7 @@ int bl_ibm_destroy(bl_ibm g)
                     g->p_model, g->p_bug, g->p_params, g->p_voff, g->p_toff, g->p_loff, g->p_poff, g->p_geom,
                     g->p_delta, g->pos, g->vel, g->force, g->ec, g->ut, g->v_pos0,
                     g->tile_count, g->tile_list, g->active, g->n_active,
-                    g->col_count, g->col_off, g->col_fill, g->col_z, g->n_hits, g->phase,
+                    g->col_bits, g->n_hits, g->phase,
                     g->flags_alt, g->force_alt, g->p_choff, g->ch_partial, g->ch_tab, g->t_vert, g->v_inc, g->v_near, g->v_blend, g->v_part, g->t_part, g->r_part,
                     g->l_part, g->ext_force, g->r_state};
     for (void* p : ptrs) hipFree(p);
@@ -3591,11 +3588,11 @@ int bl_ibm_init(bl_ibm g)
     }
     BL_HIP(hipMemset(g->tile_count, 0, L->ntiles * sizeof(int)));
     // voxelization
-    const long ncol = (long)L->nx * L->ny;
-    g->col_cap = std::max<long>(64 * g->NT, 1024);
-    if ((rc = alloc(g->col_count, ncol)) || (rc = alloc(g->col_off, ncol)) || (rc = alloc(g->col_fill, ncol)) ||
-        (rc = alloc(g->col_z, g->col_cap)) || (rc = alloc(g->n_hits, 1)) || (rc = alloc(g->phase, L->ncell)))
-        return rc;
+    const size_t nbits = (size_t)L->nx * L->ny * column_words(L->nz);
+    g->hit_cap = std::max<long>(64 * g->NT, 1024);
+    if ((rc = alloc(g->col_bits, nbits)) || (rc = alloc(g->n_hits, 1)) || (rc = alloc(g->phase, L->ncell))) return rc;
+    BL_HIP(hipMemset(g->col_bits, 0, nbits * sizeof(unsigned)));
+    BL_HIP(hipMemset(g->n_hits, 0, sizeof(int)));
     BL_HIP(hipMemset(g->phase, 0, L->ncell));
     for (auto& e : g->ev) BL_HIP(hipEventCreate(&e));
     for (auto& st : g->aux) BL_HIP(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));

@@ -138,11 +138,8 @@ struct bl_ibm_s {
     int* t_vert = nullptr;               // per triangle: its three global vertex indices
 
     // ---- voxelization ----
-    int* col_count = nullptr;
-    int* col_off = nullptr;
-    int* col_fill = nullptr;
-    double* col_z = nullptr;
-    long col_cap = 0;
+    unsigned* col_bits = nullptr;  // per (x, y) column: a toggle bit per node, then a flag word; zero between steps
+    long hit_cap = 0;              // the most hits a step may have
     int* n_hits = nullptr;
     unsigned char* phase = nullptr;
 
