@@ -937,30 +937,27 @@ __global__ void __launch_bounds__(256) k_vertex_gather(GatherArgs<R> a)
 // The progs' computeVelocity pass (staged_velocity), restricted to the
 // cells of the tiles this step's stencils touch (`touched`, the step's tile
 // flags).  `lv` carries the force field and flags of the last collision.
-// One thread per cell in z-fastest order, so population reads coalesce as
-// in the collide kernel and the staged vectors are written contiguously.
+// Where most tiles are touched, one thread per cell in z-fastest order, so
+// population reads coalesce as in the collide kernel and the staged vectors
+// are written contiguously; where few are (spread_dense), one wave per
+// touched tile off the list, since looking at every cell's flag is a launch
+// over the whole lattice (384^3 with 2 124 touched tiles: 86 us against 24).
 // (With the staging carried by the collision, k_collide_stream writes the
 // same values from the populations it loads.)
 struct StageArgs {
     LatView lv;
     const unsigned char* touched;
     void* ut;  // Vel4 of the storage's compute type
+    const int *active, *nactive;  // the touched-tile list (null: a thread per cell)
+    FastDiv dty, dtz;             // division by the tiles along y and z
 };
 
 template <class S, bool SWAPPED>
-__device__ __forceinline__ void stage_body(unsigned bx, const StageArgs& A)
+__device__ __forceinline__ void stage_cell(const StageArgs& A, unsigned c, int x, int y, int z)
 {
     using C = typename Pop<S>::C;
     using FT = typename Pop<S>::F;
     const LatView& lv = A.lv;
-    const unsigned char* __restrict__ touched = A.touched;
-    Vel4<C>* __restrict__ ut = (Vel4<C>*)A.ut;
-    const unsigned c = bx * blockDim.x + threadIdx.x;
-    if (c >= lv.ncell) return;
-    int x, y, z;
-    decode(c, lv, x, y, z);
-    const unsigned t = ((unsigned)(x >> 2) * lv.nty + (y >> 2)) * lv.ntz + (z >> 2);
-    if (!touched[t]) return;
     const unsigned char m = lv.mask ? lv.mask[c] : (unsigned char)M_FLUID;
     // the moments as the collision forms them (working form of the storage),
     // so that a staging carried by the collision gives the same values
@@ -973,11 +970,34 @@ __device__ __forceinline__ void stage_body(unsigned bx, const StageArgs& A)
         wmoments<S>(f, rb, j);
     }
     const C invRho = C(1) / (rb + C(1));
-    ut[c] = staged_velocity_m<FT, C>(lv, lv.flags, lv.force, m, c, x, y, z, j, invRho);
+    ((Vel4<C>*)A.ut)[c] = staged_velocity_m<FT, C>(lv, lv.flags, lv.force, m, c, x, y, z, j, invRho);
 }
 
 template <class S, bool SWAPPED>
-__global__ void __launch_bounds__(256) k_stage_u(StageArgs a) { stage_body<S, SWAPPED>(blockIdx.x, a); }
+__device__ __forceinline__ void stage_body(unsigned bx, unsigned nbx, const StageArgs& A)
+{
+    const LatView& lv = A.lv;
+    if (A.active) {
+        const int na = *A.nactive, lane = threadIdx.x & 63;
+        for (int a = (int)(bx * (blockDim.x >> 6) + (threadIdx.x >> 6)); a < na; a += (int)(nbx * (blockDim.x >> 6))) {
+            const unsigned t = (unsigned)A.active[a], r = fdiv(t, A.dtz), tx = fdiv(r, A.dty);
+            const int x = (int)tx * kTile + (lane >> 4), y = (int)(r - tx * lv.nty) * kTile + ((lane >> 2) & 3),
+                      z = (int)(t - r * lv.ntz) * kTile + (lane & 3);
+            if (x < lv.nx && y < lv.ny && z < lv.nz)
+                stage_cell<S, SWAPPED>(A, ((unsigned)x * lv.ny + y) * lv.nz + z, x, y, z);
+        }
+        return;
+    }
+    const unsigned c = bx * blockDim.x + threadIdx.x;
+    if (c >= lv.ncell) return;
+    int x, y, z;
+    decode(c, lv, x, y, z);
+    const unsigned t = ((unsigned)(x >> 2) * lv.nty + (y >> 2)) * lv.ntz + (z >> 2);
+    if (A.touched[t]) stage_cell<S, SWAPPED>(A, c, x, y, z);
+}
+
+template <class S, bool SWAPPED>
+__global__ void __launch_bounds__(256) k_stage_u(StageArgs a) { stage_body<S, SWAPPED>(blockIdx.x, gridDim.x, a); }
 
 // ------------------------------------------------------- interpolation
 // U_k = sum over the stencil nodes of phi(dx) phi(dy) phi(dz) u
@@ -1611,7 +1631,7 @@ __global__ void __launch_bounds__(256) k_gather_stage(GatherArgs<R> ga, int n1, 
 {
     const int bx = blockIdx.x;
     if (bx < n1) gather_body<R, GL>(ibm_block(bx, n1, ga.xcd), ga);
-    else stage_body<S, SWAPPED>(bx - n1, sa);
+    else stage_body<S, SWAPPED>(bx - n1, gridDim.x - n1, sa);
 }
 
 // Spreading (lists, weights and vertex forces) | interpolation + advection
@@ -2291,6 +2311,10 @@ StageArgs stage_args(bl_ibm g, bool spread)
     a.lv = ibm_view(g);
     a.touched = g->flags_alt;
     a.ut = g->ut;
+    a.active = spread_dense(g) ? nullptr : g->active + (long)g->last_list * L->ntiles;
+    a.nactive = g->n_active + g->last_list;
+    a.dty = make_fastdiv((unsigned)L->nty);
+    a.dtz = make_fastdiv((unsigned)L->ntz);
     if (spread) {
         a.lv.force = g->force_alt;
         if (a.lv.flags) a.lv.flags = g->flags_alt;
@@ -2299,8 +2323,14 @@ StageArgs stage_args(bl_ibm g, bool spread)
     return a;
 }
 
-// u on the cells of the touched tiles, one thread per cell
-unsigned stage_blocks(bl_ibm g) { return (unsigned)((g->lat->ncell + 255) / 256); }
+// u on the cells of the touched tiles: a thread per cell, or about a wave
+// per touched tile (at most every tile, and fewer than the vertices for a
+// membrane; a wave that finds more takes several)
+unsigned stage_blocks(bl_ibm g)
+{
+    if (spread_dense(g)) return (unsigned)((g->lat->ncell + 255) / 256);
+    return (unsigned)std::max<long>(1, std::min<long>(std::min<long>(g->lat->ntiles, g->NV) / 4 + 1, 2048));
+}
 
 template <class S>
 void launch_stage_s(const StageArgs& a, unsigned nblocks, bool swapped, hipStream_t s)
@@ -2910,7 +2940,7 @@ __global__ void __launch_bounds__(256) k_gather_stage_batch(const LayeredEntry<R
     const LayeredEntry<R>& E = tab[box];
     const int bx = (int)blockIdx.x - base[box];
     if (bx < E.ng) gather_body<R, GL>(ibm_block(bx, E.ng, E.gather.xcd), E.gather);
-    else stage_body<S, SWAPPED>(bx - E.ng, E.stage);
+    else stage_body<S, SWAPPED>(bx - E.ng, E.nst, E.stage);
 }
 
 template <class S, int SW, class R>
