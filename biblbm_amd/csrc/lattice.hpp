@@ -2,6 +2,7 @@
 // in-place AA pattern, cell mask, tile-gated external force, phase.
 #pragma once
 
+#include <mutex>
 #include <vector>
 
 #include "common.hpp"
@@ -78,6 +79,8 @@ struct bl_lattice_s {
 
     // scratch
     double* d_stage = nullptr;  // ncell * 19 doubles, allocated on demand
+    double* d_read = nullptr;   // bl_lattice_get_moments: ncell * 4 doubles, allocated on demand (kReadKept)
+    std::mutex read_lock;       // d_read is one reader's at a time
     double* d_partials = nullptr;
     long nwall = 0;
     bl_ibm ibm = nullptr;
