@@ -919,11 +919,11 @@ __global__ void __launch_bounds__(256) k_vertex_gather(GatherArgs<R> a)
 // The progs' computeVelocity pass (staged_velocity), restricted to the
 // cells of the tiles this step's stencils touch (`touched`, the step's tile
 // flags).  `lv` carries the force field and flags of the last collision.
-// Where most tiles are touched, one thread per cell in z-fastest order, so
-// population reads coalesce as in the collide kernel and the staged vectors
-// are written contiguously; where few are (spread_dense), one wave per
-// touched tile off the list, since looking at every cell's flag is a launch
-// over the whole lattice (384^3 with 2 124 touched tiles: 86 us against 24).
+// One thread per cell in z-fastest order, so population reads coalesce as
+// in the collide kernel and the staged vectors are written contiguously; or,
+// where few tiles of many are touched (stage_by_list), one wave per touched
+// tile off the list, since looking at every cell's flag is a launch over the
+// whole lattice (384^3 with 2 124 touched tiles: 86 us against 24).
 // (With the staging carried by the collision, k_collide_stream writes the
 // same values from the populations it loads.)
 struct StageArgs {
@@ -2286,6 +2286,12 @@ LatView ibm_view(bl_ibm g)
     return lv;
 }
 
+// Where the staging takes the touched tiles off their list: few of many
+// tiles.  The list costs two dependent loads before a wave's tile is known
+// (24^3: staging 4.2 -> 6.0 us; 64^3 beside the gather 5.3 -> 5.5), the cells
+// a workgroup per 256 (257 x 67 x 67: 7.5 us against 7.3, 384^3 86 against 24).
+bool stage_by_list(bl_ibm g) { return !spread_dense(g) && g->lat->ncell >= 1l << 20; }
+
 // Velocity staging of the step whose binning is the last one.  Before that
 // binning's spreading (`spread` false) the last collision's force field and
 // flags are the lattice's, and the binning's flags are in flags_alt; after
@@ -2297,7 +2303,7 @@ StageArgs stage_args(bl_ibm g, bool spread)
     a.lv = ibm_view(g);
     a.touched = g->flags_alt;
     a.ut = g->ut;
-    a.active = spread_dense(g) ? nullptr : g->active + (long)g->last_list * L->ntiles;
+    a.active = stage_by_list(g) ? g->active + (long)g->last_list * L->ntiles : nullptr;
     a.nactive = g->n_active + g->last_list;
     a.dty = make_fastdiv((unsigned)L->nty);
     a.dtz = make_fastdiv((unsigned)L->ntz);
@@ -2314,7 +2320,7 @@ StageArgs stage_args(bl_ibm g, bool spread)
 // membrane; a wave that finds more takes several)
 unsigned stage_blocks(bl_ibm g)
 {
-    if (spread_dense(g)) return (unsigned)((g->lat->ncell + 255) / 256);
+    if (!stage_by_list(g)) return (unsigned)((g->lat->ncell + 255) / 256);
     return (unsigned)std::max<long>(1, std::min<long>(std::min<long>(g->lat->ntiles, g->NV) / 4 + 1, 2048));
 }
 
