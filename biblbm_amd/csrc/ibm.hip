@@ -2564,18 +2564,45 @@ void launch_gather(bl_ibm g, hipStream_t s, bool walls)
     hipLaunchKernelGGL((k_vertex_gather<R, GL>), dim3(nblk(GL * g->NV)), dim3(256), 0, s, gather_args<R>(g, walls));
 }
 
-void launch_membrane(bl_ibm g, hipStream_t s, bool walls)
+void launch_vertex_forces(bl_ibm g, hipStream_t s, bool walls)
 {
-    const int eb = g->lp[BL_IBM_ELEM_BLOCK];
     with_vreal(g, [&](auto tag) {
         using R = decltype(tag);
-        hipLaunchKernelGGL(k_elem_forces<R>, dim3(nblk(g->NT + g->NP + g->NL, eb)), dim3(eb), 0, s, elem_args<R>(g));
         const int gl = g->lp[BL_IBM_GATHER_LANES];
         if (gl == 2) launch_gather<R, 2>(g, s, walls);
         else if (gl == 8) launch_gather<R, 8>(g, s, walls);
         else launch_gather<R, 4>(g, s, walls);
         return 0;
     });
+}
+
+void launch_membrane(bl_ibm g, hipStream_t s, bool walls)
+{
+    const int eb = g->lp[BL_IBM_ELEM_BLOCK];
+    with_vreal(g, [&](auto tag) {
+        using R = decltype(tag);
+        hipLaunchKernelGGL(k_elem_forces<R>, dim3(nblk(g->NT + g->NP + g->NL, eb)), dim3(eb), 0, s, elem_args<R>(g));
+        return 0;
+    });
+    launch_vertex_forces(g, s, walls);
+}
+
+// binning | membrane element forces, one launch
+int bin_elem_launch(bl_ibm g, hipStream_t s)
+{
+    int rc;
+    if (!g->prepped && (rc = prep_bin(g, s))) return rc;
+    g->prepped = false;
+    with_vreal(g, [&](auto tag) {
+        using R = decltype(tag);
+        const int bb = g->lp[BL_IBM_BIN_BLOCK];  // both halves of the paired launch
+        const int nb = bin_blocks(g, bb, 1), ne = (int)nblk(g->NT + g->NP + g->NL, bb);
+        hipLaunchKernelGGL(k_bin_elem<R>, dim3(nb + ne), dim3(bb), 0, s, bin_args<R>(g), nb, elem_args<R>(g));
+        return 0;
+    });
+    BL_CHECK_LAUNCH();
+    binned(g);
+    return BL_OK;
 }
 
 int do_forces(bl_ibm g, hipStream_t s)
@@ -2724,13 +2751,27 @@ int step_forked(bl_ibm g)
 // Whether coupled steps carry the velocity staging in the collision
 // (step_fused).  Only without a phase field: the collision of a step reads
 // the phase voxelized from the moved vertices, which need the staged
-// velocity first.  By default for 65 536 vertices or more, where the
-// staging pass reads populations over most of the lattice.
-bool use_fused(bl_ibm g)
+// velocity first.  By default for kPairedVertices vertices or more ...
+bool fused_large(bl_ibm g)
 {
     bl_lattice L = g->lat;
     if (g->fused_staging == 0 || g->NV == 0 || L->omega_c0 != L->omega_c1) return false;
-    return g->fused_staging == 1 || g->NV >= 65536;
+    return g->fused_staging == 1 || g->NV >= kPairedVertices;
+}
+
+// ... and, outside batches of boxes, for fewer where most tiles of a lattice
+// of kStagedBytes of populations are staged: the pass that the collision
+// saves reads them all again (171 x 70 x 101 FP64, 184 MB: 39 us beside the
+// gather, 10 more in the collision; 223 -> 213 us a step), and the two stages
+// it would have shared launches with cost about 15 us by themselves, what
+// the pass takes over some 70 MB.
+constexpr size_t kStagedBytes = 96u << 20;
+bool use_fused(bl_ibm g)
+{
+    bl_lattice L = g->lat;
+    if (fused_large(g)) return true;
+    return g->fused_staging < 0 && g->layered < 0 && g->NV > 0 && L->omega_c0 == L->omega_c1 && spread_dense(g) &&
+           (size_t)Q * L->stride * L->pop_bytes >= kStagedBytes;
 }
 
 // One coupled step with the velocity staging carried by the collision.
@@ -2742,6 +2783,8 @@ bool use_fused(bl_ibm g)
 //      stages u (pre-collision populations, the last collision's force
 //      field) on the touched tiles; post-stream walls; interpolation +
 //      advection (readying the next binning's list); geometry.
+// (With few vertices A is on M too, the element forces in the binning's
+// launch.)
 // The staged values are those of k_stage_u; one pass over the touched
 // populations is saved.
 int step_fused(bl_ibm g)
@@ -2750,12 +2793,18 @@ int step_fused(bl_ibm g)
     bl_lattice L = g->lat;
     hipStream_t M = L->stream, A = g->aux[0];
     hipEvent_t* e = g->fev;
-    BL_HIP(hipEventRecord(e[0], M));
-    BL_HIP(hipStreamWaitEvent(A, e[0], 0));
-    if ((rc = do_forces(g, A))) return rc;
-    BL_HIP(hipEventRecord(e[1], A));
-    if ((rc = do_bin(g, M))) return rc;
-    BL_HIP(hipStreamWaitEvent(M, e[1], 0));
+    if (use_pairs(g)) {
+        if (!g->pp.empty() && (rc = interactions_launch(g, M))) return rc;
+        if ((rc = bin_elem_launch(g, M))) return rc;
+        launch_vertex_forces(g, M, true);
+    } else {
+        BL_HIP(hipEventRecord(e[0], M));
+        BL_HIP(hipStreamWaitEvent(A, e[0], 0));
+        if ((rc = do_forces(g, A))) return rc;
+        BL_HIP(hipEventRecord(e[1], A));
+        if ((rc = do_bin(g, M))) return rc;
+        BL_HIP(hipStreamWaitEvent(M, e[1], 0));
+    }
     if ((rc = launch_spread(g, M))) return rc;
     // after the swap: the lattice holds this step's field and flags (the
     // touched tiles), the boundary's spare buffers the last collision's
@@ -2806,12 +2855,7 @@ int step_layered_s(bl_ibm g)
     if ((rc = vreal_matches_storage(g))) return rc;
     hipStream_t s = L->stream;
     if (!g->pp.empty() && (rc = interactions_launch(g, s))) return rc;
-    if (!g->prepped && (rc = prep_bin(g, s))) return rc;
-    g->prepped = false;
-    const int bb = g->lp[BL_IBM_BIN_BLOCK];  // both halves of the paired launch
-    const int nb = bin_blocks(g, bb, 1), ne = (int)nblk(g->NT + g->NP + g->NL, bb);
-    hipLaunchKernelGGL(k_bin_elem<R>, dim3(nb + ne), dim3(bb), 0, s, bin_args<R>(g), nb, elem_args<R>(g));
-    binned(g);
+    if ((rc = bin_elem_launch(g, s))) return rc;
     const int gl = g->lp[BL_IBM_GATHER_LANES];
     if (gl == 2) launch_gather_stage<S, R, 2>(g, s);
     else if (gl == 8) launch_gather_stage<S, R, 8>(g, s);
@@ -2887,7 +2931,7 @@ struct LayeredEntry {
 bool layered_batchable(bl_ibm g)
 {
     const bl_lattice L = g->lat;
-    return L && g->inited && g->NV > 0 && use_layered(g) && !use_fused(g) && g->pp.empty() &&
+    return L && g->inited && g->NV > 0 && use_layered(g) && !fused_large(g) && g->pp.empty() &&
            L->omega_c0 == L->omega_c1 && !g->bins_dirty && !g->alt_full && !ibm_needs_settle(g) && !g->timing &&
            g->n_rigid == 0 && g->vreal == (L->storage == BL_STORE_F64 ? 8 : 4);
 }
