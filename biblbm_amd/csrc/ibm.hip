@@ -157,7 +157,12 @@ __device__ __forceinline__ int node_at(int bw, int k, int n, int per)
 // wrap), kept in registers.
 struct AxisTiles {
     int t0 = -1, t1 = -1, t2 = -1, m = 0;
-    __device__ __forceinline__ int get(int i) const { return i == 0 ? t0 : (i == 1 ? t1 : t2); }
+    // by masks: as a choice of fields they became indexed loads from scratch
+    __device__ __forceinline__ int get2(int i) const { return t0 ^ ((t0 ^ t1) & -i); }  // i 0 or 1
+    __device__ __forceinline__ int get(int i) const
+    {
+        return t0 ^ ((t0 ^ t1) & -(int)(i == 1)) ^ ((t0 ^ t2) & -(int)(i == 2));
+    }
 };
 
 __device__ __forceinline__ AxisTiles axis_tiles(int bw, int S, int n, int per)
@@ -256,6 +261,12 @@ struct StencilTiles {
     {
         if (i >= ax[0].m || j >= ax[1].m || k >= ax[2].m) return -1;
         return (ax[0].get(i) * gd.nt[1] + ax[1].get(j)) * gd.nt[2] + ax[2].get(k);
+    }
+    // the same for i, j, k of 0 or 1
+    __device__ __forceinline__ int at2(const Grid& gd, int i, int j, int k) const
+    {
+        if (i >= ax[0].m || j >= ax[1].m || k >= ax[2].m) return -1;
+        return (ax[0].get2(i) * gd.nt[1] + ax[1].get2(j)) * gd.nt[2] + ax[2].get2(k);
     }
     __device__ __forceinline__ bool wide() const { return ax[0].m > 2 || ax[1].m > 2 || ax[2].m > 2; }
 };
@@ -403,7 +414,7 @@ __device__ __forceinline__ int count_pair(const BinArgs<R>& A, const StencilTile
     // tiles past the 2 x 2 x 2 product: a third one on an axis (a wrap at a
     // size that is no multiple of 4), and a full table
     int direct = -1;
-    const int t = st.at(A.gd, r >> 2, (r >> 1) & 1, r & 1);
+    const int t = st.at2(A.gd, r >> 2, (r >> 1) & 1, r & 1);
     int code = -1;
     if (t >= 0) {
         const int sl = hash_insert(keys, t);
@@ -1709,9 +1720,9 @@ __global__ void k_move(long NV, R* __restrict__ pos, const R* __restrict__ vel)
 // particles all have at most kGeomTriangles triangles take one launch of a
 // workgroup per particle instead (k_geom: a lane's triangles one after the
 // other, a butterfly per wave, the waves in order).  Both wait for memory:
-// 1 280 triangles take 6.2 us in one launch, 4.5 + 4.6 in two, but 5 120
-// take 14 (each lane ten deep) against 9.1, and 400 cells of both sizes 22
-// against 16.
+// 1 280 triangles take 5.9 us in one launch, 4.5 + 4.6 in two, but 5 120
+// take 13 (with 512 or 1 024 lanes alike) against 9.2, and 18 cells of them
+// 17 against 9.9.
 constexpr long kGeomTriangles = 2048;
 template <class R>
 struct GeomArgs {
