@@ -281,7 +281,9 @@ int bl_ibm_tile_stats(bl_ibm g, long long out[2]);
  * computeVelocity pass, restricted to the touched tiles) in the
  * collide-and-stream launch, which then runs before the interpolation and
  * advection of the same step; 0 stages in a pass of its own before the
- * spreading; -1 (default) picks 1 for 65 536 vertices or more.  Without a
+ * spreading; -1 (default) picks 1 for 65 536 vertices or more, and, with
+ * bl_ibm_set_layered at its default too, where the vertices outnumber the
+ * 4x4x4 tiles of a lattice of 96 MiB of populations or more.  Without a
  * phase field only (omega_in == omega_out); otherwise the separate pass is
  * used.  The staged values are the same either way. */
 int bl_ibm_set_fused_staging(bl_ibm g, int mode);
