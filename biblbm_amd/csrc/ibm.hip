@@ -206,14 +206,23 @@ __device__ __forceinline__ int stencil_base(int first, int n, int per)
 // (Peskin) and 1 + r, r, 1 - r (Roma) with r = x - (first + 1), and phi's
 // square roots at all of them are the one at r: 1 + 4 r (1 - r) and
 // 1 - 3 r^2.  In registers by name: an indexed array here went to scratch.
+// The kernel is the stencil's width SW (Peskin 4, Roma 3, top hat 2) at
+// compile time: of a run-time choice among the three the compiler made code
+// that left the top hat's first weight unset.
 template <class R>
 struct W4 {
     R w0, w1, w2, w3;
 };
 
-template <class R>
-__device__ __forceinline__ W4<R> axis_weights(int kernel, R x, int first)
+__host__ __device__ constexpr int kernel_of(int SW)
 {
+    return SW == 4 ? BL_KERNEL_PESKIN : (SW == 3 ? BL_KERNEL_ROMA : BL_KERNEL_TOPHAT);
+}
+
+template <int SW, class R>
+__device__ __forceinline__ W4<R> axis_weights(R x, int first)
+{
+    constexpr int kernel = kernel_of(SW);
     const R r = x - (R)(first + 1);
     if (kernel == BL_KERNEL_PESKIN) {
         const R q = sqrt(R(1) + R(4) * r * (R(1) - r));
@@ -1033,7 +1042,6 @@ template <class R>
 struct InterpArgs {
     Grid gd;
     long NV;
-    int kernel;
     double h;
     const Vel4<R>* vp;  // the binning's position copies
     const void* ut;     // Vel4<C>
@@ -1053,6 +1061,7 @@ __device__ __forceinline__ void interp_body(long bx, int nbx, const InterpArgs<R
     R* __restrict__ pos = A.pos;
     const NearView<R>& nw = A.nw;
     if (A.lr.act) list_reset(A.lr, (int)bx, nbx);  // the next binning's list, carried by this launch
+    constexpr int kernel = kernel_of(SW);
     constexpr int LA = SW == 2 ? 2 : 4;
     constexpr int LPV = LA * LA;
     const long gid = ibm_block(bx, nbx, A.xcd) * blockDim.x + threadIdx.x;
@@ -1068,11 +1077,11 @@ __device__ __forceinline__ void interp_body(long bx, int nbx, const InterpArgs<R
     R wx[SW], wy, wz;
     if (SW == 2) {
 #pragma unroll
-        for (int i = 0; i < SW; ++i) wx[i] = dirac<R>(A.kernel, (R)(fx + i) - P.x);
-        wy = dirac<R>(A.kernel, (R)(fy + j) - P.y);
-        wz = dirac<R>(A.kernel, (R)(fz + k) - P.z);
+        for (int i = 0; i < SW; ++i) wx[i] = dirac<R>(kernel, (R)(fx + i) - P.x);
+        wy = dirac<R>(kernel, (R)(fy + j) - P.y);
+        wz = dirac<R>(kernel, (R)(fz + k) - P.z);
     } else {
-        const R mine = dirac<R>(A.kernel, (j == 0 ? (R)(fx + k) - P.x : (j == 1 ? (R)(fy + k) - P.y : (R)(fz + k) - P.z)));
+        const R mine = dirac<R>(kernel, (j == 0 ? (R)(fx + k) - P.x : (j == 1 ? (R)(fy + k) - P.y : (R)(fz + k) - P.z)));
 #pragma unroll
         for (int i = 0; i < SW; ++i) wx[i] = __shfl(mine, i, LPV);
         wy = __shfl(mine, 4 + j, LPV);
@@ -1235,7 +1244,7 @@ template <class R>
 struct SpreadArgs {
     LatView lv;
     Grid gd;
-    int kernel, Sw, n_small;
+    int n_small;
     double h;
     // the touched-tile list (null: every tile is looked at, in space order)
     const int *active, *nactive, *big, *nbig;
@@ -1283,7 +1292,7 @@ __device__ __forceinline__ Entry<R> load_entry(const SpreadArgs<R>& A, int e)
 
 // Its weights on the tile's cells (rows 0-11: axis-major, 4 cells per axis)
 // and its force (rows 12-14).
-template <class R>
+template <int SW, class R>
 __device__ __forceinline__ void entry_weights(const SpreadArgs<R>& A, const int org[3], const Entry<R>& E, R ev[15])
 {
     const Grid& gd = A.gd;
@@ -1293,9 +1302,9 @@ __device__ __forceinline__ void entry_weights(const SpreadArgs<R>& A, const int 
     for (int ax = 0; ax < 3; ++ax) {
         const int first = stencil_first(x[ax], h);
         const int b = stencil_base(first, gd.n[ax], gd.per[ax]);
-        W4<R> w = axis_weights<R>(A.kernel, x[ax], first);
+        W4<R> w = axis_weights<SW, R>(x[ax], first);
         if (A.nw.on) {
-            const W4<R> t = axis_weights<R>(BL_KERNEL_TOPHAT, x[ax], first);
+            const W4<R> t = axis_weights<2, R>(x[ax], first);
             w = {E.top ? t.w0 : w.w0, E.top ? t.w1 : w.w1, E.top ? t.w2 : w.w2, E.top ? t.w3 : w.w3};
         }
         // the tile's first node past the stencil's; a stencil that wrapped
@@ -1339,7 +1348,7 @@ __device__ __forceinline__ void chunk_sum(const R (*ew)[kChunkRow], int cnt, int
 
 // Adds the sorted entries [lo, hi) of a tile to acc, 64 at a time; key(e)
 // gives the e-th sorted entry.
-template <class R, class KeyOf>
+template <int SW, class R, class KeyOf>
 __device__ __forceinline__ void sum_entries(const SpreadArgs<R>& A, const int org[3], int lo, int hi, KeyOf key,
                                             R (*ew)[kChunkRow], int lane, typename TileSum<R>::V& acc)
 {
@@ -1348,7 +1357,7 @@ __device__ __forceinline__ void sum_entries(const SpreadArgs<R>& A, const int or
         R ev[15];
 #pragma unroll
         for (int r = 0; r < 15; ++r) ev[r] = R(0.0);
-        if (e < hi) entry_weights<R>(A, org, load_entry<R>(A, key(e)), ev);
+        if (e < hi) entry_weights<SW, R>(A, org, load_entry<R>(A, key(e)), ev);
 #pragma unroll
         for (int half = 0; half < 2; ++half) {
             const int cnt = min(kChunk, hi - c0 - half * kChunk);
@@ -1433,7 +1442,7 @@ __device__ __forceinline__ int rank_in_run(const int* r, int key)
     return lo + (r[lo] < key ? 1 : 0);
 }
 
-template <class FT, class R>
+template <class FT, int SW, class R>
 __device__ __forceinline__ void spread_small(int blk, int nb, int* keys, R (*ew_all)[15][kChunkRow],
                                              const SpreadArgs<R>& A)
 {
@@ -1474,7 +1483,7 @@ __device__ __forceinline__ void spread_small(int blk, int nb, int* keys, R (*ew_
             tile_origin<R>(A, t, org);
             const R g = column_start<R>(A.lv, lane);
             typename TileSum<R>::V acc = {g, g, g, g};
-            sum_entries<R>(A, org, 0, n, [&](int e) { return k[e]; }, ew, lane, acc);
+            sum_entries<SW, R>(A, org, 0, n, [&](int e) { return k[e]; }, ew, lane, acc);
             store_tile<FT, R>(A.lv, gd, org, lane, acc, (FT*)A.Fout);
             if (lane == 0) count[t] = 0;
         } else if (n > 0 && n <= 64) {
@@ -1493,7 +1502,7 @@ __device__ __forceinline__ void spread_small(int blk, int nb, int* keys, R (*ew_
             const int col = live ? rank : lane;
             if (!live) E.F[0] = E.F[1] = E.F[2] = R(0);
             R ev[15];
-            entry_weights<R>(A, org, E, ev);
+            entry_weights<SW, R>(A, org, E, ev);
             for (int h0 = 0; h0 < n; h0 += kChunk) {
                 if ((col & ~(kChunk - 1)) == h0)
 #pragma unroll
@@ -1510,7 +1519,7 @@ __device__ __forceinline__ void spread_small(int blk, int nb, int* keys, R (*ew_
     }
 }
 
-template <class FT, class R>
+template <class FT, int SW, class R>
 __device__ __forceinline__ void spread_big(int blk, int nb, int* keys, int* runs, R (*ew_all)[15][kChunkRow],
                                            R (*part)[4][64], const SpreadArgs<R>& A)
 {
@@ -1568,7 +1577,7 @@ __device__ __forceinline__ void spread_big(int blk, int nb, int* keys, int* runs
         const int q = (n + kSpreadWaves - 1) / kSpreadWaves;
         const int lo = min(n, wv * q), hi = min(n, lo + q);
         typename TileSum<R>::V acc = {R(0), R(0), R(0), R(0)};
-        sum_entries<R>(A, org, lo, hi, [&](int k) { return keys[k]; }, ew, lane, acc);
+        sum_entries<SW, R>(A, org, lo, hi, [&](int k) { return keys[k]; }, ew, lane, acc);
 #pragma unroll
         for (int r = 0; r < 4; ++r) part[wv][r][lane] = acc[r];
         __syncthreads();
@@ -1586,7 +1595,7 @@ __device__ __forceinline__ void spread_big(int blk, int nb, int* keys, int* runs
     }
 }
 
-template <class S, class R>
+template <class S, int SW, class R>
 __device__ __forceinline__ void spread_body(int bx, int nbx, const SpreadArgs<R>& A)
 {
     using FT = typename Pop<S>::F;
@@ -1594,14 +1603,14 @@ __device__ __forceinline__ void spread_body(int bx, int nbx, const SpreadArgs<R>
     __shared__ int runs[64 * kSpreadWaves];
     __shared__ R ew_all[kSpreadWaves][15][kChunkRow];
     __shared__ R part[kSpreadWaves][4][64];
-    if (bx < A.n_small) spread_small<FT, R>((int)ibm_block(bx, A.n_small, A.xcd), A.n_small, keys, ew_all, A);
-    else spread_big<FT, R>(bx - A.n_small, nbx - A.n_small, keys, runs, ew_all, part, A);
+    if (bx < A.n_small) spread_small<FT, SW, R>((int)ibm_block(bx, A.n_small, A.xcd), A.n_small, keys, ew_all, A);
+    else spread_big<FT, SW, R>(bx - A.n_small, nbx - A.n_small, keys, runs, ew_all, part, A);
 }
 
-template <class S, class R>
+template <class S, int SW, class R>
 __global__ void __launch_bounds__(64 * kSpreadWaves) k_spread(SpreadArgs<R> a)
 {
-    spread_body<S, R>(blockIdx.x, gridDim.x, a);
+    spread_body<S, SW, R>(blockIdx.x, gridDim.x, a);
 }
 
 // ------------------------------------------- stages paired in one launch
@@ -1634,7 +1643,7 @@ template <class S, int SW, class R>
 __global__ void __launch_bounds__(256) k_spread_interp(SpreadArgs<R> sp, int n1, InterpArgs<R> ia)
 {
     const int bx = blockIdx.x;
-    if (bx < n1) spread_body<S, R>(bx, n1, sp);
+    if (bx < n1) spread_body<S, SW, R>(bx, n1, sp);
     else interp_body<typename Pop<S>::C, SW, true, R>(bx - n1, (int)gridDim.x - n1, ia);
 }
 
@@ -2367,7 +2376,6 @@ InterpArgs<R> interp_args(bl_ibm g, const ListReset& lr)
 {
     InterpArgs<R> a;
     a.gd = grid_of(g->lat);
-    a.kernel = g->kernel;
     a.h = g->h;
     a.NV = g->NV;
     a.vp = (const Vel4<R>*)g->v_pos0;
@@ -2434,8 +2442,6 @@ SpreadArgs<R> spread_args(bl_ibm g, unsigned& blocks, int share = 1)
     SpreadArgs<R> a;
     a.lv = ibm_view(g);
     a.gd = grid_of(L);
-    a.kernel = g->kernel;
-    a.Sw = g->S;
     a.h = g->h;
     const bool dense = spread_dense(g);
     a.small = dense ? kSmallTile : kSparseTile;
@@ -2487,21 +2493,25 @@ void spread_swap(bl_ibm g)
     g->bins_dirty = false;
 }
 
+template <class S, class R>
+void launch_spread_s(bl_ibm g, hipStream_t s)
+{
+    unsigned nb;
+    const SpreadArgs<R> a = spread_args<R>(g, nb);
+    if (g->S == 4) hipLaunchKernelGGL((k_spread<S, 4, R>), dim3(nb), dim3(256), 0, s, a);
+    else if (g->S == 3) hipLaunchKernelGGL((k_spread<S, 3, R>), dim3(nb), dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((k_spread<S, 2, R>), dim3(nb), dim3(256), 0, s, a);
+}
+
 int launch_spread(bl_ibm g, hipStream_t s)
 {
-    bl_lattice L = g->lat;
     if (g->NV == 0) return BL_OK;
     int rc = vreal_matches_storage(g);
     if (rc) return rc;
-    unsigned nb;
-    if (L->storage == BL_STORE_F64) {
-        const SpreadArgs<double> a = spread_args<double>(g, nb);
-        hipLaunchKernelGGL((k_spread<double, double>), dim3(nb), dim3(256), 0, s, a);
-    } else {
-        const SpreadArgs<float> a = spread_args<float>(g, nb);
-        if (L->storage == BL_STORE_F32) hipLaunchKernelGGL((k_spread<float, float>), dim3(nb), dim3(256), 0, s, a);
-        else hipLaunchKernelGGL((k_spread<__half, float>), dim3(nb), dim3(256), 0, s, a);
-    }
+    const int st = g->lat->storage;
+    if (st == BL_STORE_F64) launch_spread_s<double, double>(g, s);
+    else if (st == BL_STORE_F32) launch_spread_s<float, float>(g, s);
+    else launch_spread_s<__half, float>(g, s);
     BL_CHECK_LAUNCH();
     spread_swap(g);
     return BL_OK;
@@ -3021,7 +3031,7 @@ __global__ void __launch_bounds__(256) k_spread_interp_batch(const LayeredEntry<
     const int box = batch_box(base, nbox, (int)blockIdx.x);
     const LayeredEntry<R>& E = tab[box];
     const int bx = (int)blockIdx.x - base[box];
-    if (bx < E.nsp) spread_body<S, R>(bx, E.nsp, E.spread);
+    if (bx < E.nsp) spread_body<S, SW, R>(bx, E.nsp, E.spread);
     else interp_body<typename Pop<S>::C, SW, true, R>(bx - E.nsp, E.nip, E.interp);
 }
 
