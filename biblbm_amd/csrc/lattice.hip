@@ -442,26 +442,38 @@ bool zseg_ok(const bl_lattice_s* L, int B)
 // The launch shape of a lattice that nobody tuned, by the bytes of its
 // populations against the 256 MiB last-level cache (the pass is bound by
 // memory; 4 GiB copy on the same card: 6.17 TB/s).  Ratios are against one
-// contiguous range of blocks per XCD without hints (order 1), even / odd
-// step, over cubes and channels of 64^3 to 384^3:
-//   fewer than 2^19 cells: order 1.  Chunks leave XCDs without work (64^3
-//     in chunks of 64: 0.96 / 0.94).
-//   in the cache: chunks of 256 blocks, so that the eight XCDs stream from
-//     nearby planes and a neighbour's row is read while it is still there:
-//     120 x 100 x 133 FP64 1.12 / 1.05, FP32 1.06 / 1.12, FP16s 1.15 / 1.25;
-//     hints lose there (0.6-0.9), they bypass the cache that holds it all.
-//   beyond it: chunks of 64 (FP64 201 x 199 x 181 1.16 / 1.07, FP32 1.13 /
-//     1.07, FP16s 1.12 / 0.97); even steps of FP64 and FP32 lattices whose
-//     planes start at multiples of 1 MiB, or beyond 2 GiB, stream past the
-//     cache instead, chunks of 16 (384^3 FP64 1.09 against 1.02, 256^3 FP32
-//     1.13 against 1.01: equally aligned planes compete for the same sets);
-//     FP64 odd steps take 128-cell z-segments, z-aligned and so whole-line
-//     streaming stores, where nz allows (256^3 1.08, 384^3 1.05).
+// contiguous range of blocks per XCD without hints (order 1) on both
+// parities, over whole runs of steps of periodic boxes and channels (a
+// launch timed between others of other shapes misses what the step before
+// left in the caches):
+//   in the cache: order 1.  Each XCD then meets the cells that it had a step
+//     before; chunks of 256 blocks lose over the whole range (FP16s 39 x 74 x
+//     185 0.93, 30 x 206 x 137 0.90, 526 x 47 x 175 0.98; FP32 108 x 83 x 83
+//     0.97, 225 x 85 x 180 0.98; FP64 50 x 224 x 81 0.98), hints more
+//     (0.6-0.9: they bypass the cache that holds it all).
+//   up to 4/3 of it: odd steps deal chunks of 64, so that they do not start
+//     where the even ones' first rows have been pushed out (FP16s 198 x 159 x
+//     238 1.30, 274 x 230 x 125 1.07; FP32 395 x 111 x 103 1.08; FP64 44 x 183
+//     x 257 1.00, 128 x 95 x 185 1.07; chunks on both parities 1.22, 0.97,
+//     1.01, 0.95, 0.98), but order 1 on both where planes start at multiples
+//     of 256 KiB and compete for the same sets (FP16s 672 x 192 x 64 0.92 in
+//     chunks, FP64 128^3 0.95, with hints 0.88).
+//   beyond: chunks of 64 on both (FP16s 240 x 232 x 224 1.10, 375 MiB and
+//     more 1.00-1.16; FP32 204 x 200 x 181 1.11, 381 x 175 x 83 1.02; FP64
+//     301 x 129 x 181 1.04, 88 x 192 x 160 1.02).  Even steps of FP64 and FP32
+//     lattices whose planes start at multiples of 1 MiB, or beyond 2 GiB,
+//     stream past the cache instead, chunks of 16 (384^3 FP64 1.09 against
+//     1.02, 256^3 FP32 1.13 against 1.01); FP64 odd steps take 128-cell
+//     z-segments, z-aligned and so whole-line streaming stores, where nz
+//     allows (256^3 1.08, 384^3 1.05).
 //   beyond it and carrying the velocity staging: the hints keep the vertex
 //     data, the force field and the staged velocities in the cache (512 x
 //     128 x 128 with 400 cells, FP32: even step 0.312 -> 0.235 ms, odd 0.315
 //     -> 0.27 ms in z-segments, -> 0.285 ms per cell; FP16s even 0.176 ->
-//     0.154 ms, odd no gain).
+//     0.154 ms, odd no gain).  In the cache, from 2^19 cells, chunks of 256:
+//     171 x 70 x 101 FP64 with 46 000 vertices 181 -> 174 us a coupled step,
+//     200 x 100 x 120 FP32 with 71 000 172 -> 168, 128^3 FP32 with 96 000
+//     164 -> 166.
 void auto_launch(const bl_lattice_s* L, bool odd, bool emit, int& block, int& order, int& nt)
 {
     constexpr size_t kCache = 256ull << 20;
@@ -470,9 +482,12 @@ void auto_launch(const bl_lattice_s* L, bool odd, bool emit, int& block, int& or
     block = 256;
     order = 1;
     nt = 0;
-    if (L->ncell < (1L << 19)) return;
     if (bytes <= kCache) {
-        order = 256;
+        if (emit && L->ncell >= (1L << 19)) order = 256;
+        return;
+    }
+    if (!emit && bytes <= kCache / 3 * 4) {
+        if (odd && plane % (256u << 10) != 0) order = 64;
         return;
     }
     order = 64;

@@ -13,12 +13,17 @@ def _state(L, rng):
 
 
 @pytest.mark.parametrize("storage,shape,even,odd", [
-    ("f32", (64, 64, 127), (256, 1, 0), (256, 1, 0)),          # below 2^19 cells
-    ("f32", (64, 64, 128), (256, 256, 0), (256, 256, 0)),      # in the cache
-    ("f64", (131, 128, 127), (256, 64, 0), (256, 64, 0)),      # beyond it
-    ("f64", (128, 128, 128), (256, 16, 1), (-128, 64, 1)),     # and with equally aligned planes, whole z-segments
-    ("f32", (224, 128, 128), (256, 16, 1), (256, 64, 0)),
-    ("f16s", (432, 128, 128), (256, 64, 0), (256, 64, 0)),
+    ("f32", (64, 64, 127), (256, 1, 0), (256, 1, 0)),          # in the cache: each XCD keeps its range
+    ("f32", (64, 64, 128), (256, 1, 0), (256, 1, 0)),
+    ("f64", (128, 111, 124), (256, 1, 0), (256, 1, 0)),
+    ("f64", (131, 128, 127), (256, 1, 0), (256, 64, 0)),       # up to 4/3 of it
+    ("f16s", (437, 128, 127), (256, 1, 0), (256, 64, 0)),
+    ("f64", (128, 128, 128), (256, 1, 0), (256, 1, 0)),        # with equally aligned planes
+    ("f32", (224, 128, 128), (256, 1, 0), (256, 1, 0)),
+    ("f16s", (432, 128, 128), (256, 1, 0), (256, 1, 0)),
+    ("f16s", (580, 128, 127), (256, 64, 0), (256, 64, 0)),     # beyond
+    ("f64", (144, 128, 128), (256, 16, 1), (-128, 64, 1)),     # with equally aligned planes, whole z-segments
+    ("f32", (288, 128, 128), (256, 16, 1), (256, 64, 0)),
 ])
 def test_untuned_shapes_by_size(device, storage, shape, even, odd):
     from biblbm_amd.lattice import Lattice, BOUNCE_BACK
