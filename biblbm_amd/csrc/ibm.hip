@@ -2311,11 +2311,20 @@ LatView ibm_view(bl_ibm g)
     return lv;
 }
 
-// Where the staging takes the touched tiles off their list: few of many
-// tiles.  The list costs two dependent loads before a wave's tile is known
-// (24^3: staging 4.2 -> 6.0 us; 64^3 beside the gather 5.3 -> 5.5), the cells
-// a workgroup per 256 (257 x 67 x 67: 7.5 us against 7.3, 384^3 86 against 24).
-bool stage_by_list(bl_ibm g) { return !spread_dense(g) && g->lat->ncell >= 1l << 20; }
+// Where the staging takes the touched tiles off their list: few of many.
+// By cells, every cell looks at its tile's flag (1.6 us for 10^6 cells) and
+// the touched ones load whole lines; off the list a wave loads a tile's 4 x
+// 4 rows of 4, a part of each line, 1.5 to 4.5 ns a tile more.  Steps with
+// NV vertices per tile, by cells | off the list: 384^3 FP64 0.01, the pass
+// alone 86 | 24 us; 300 x 200 x 190 0.11 FP64 784 | 775, FP16s 260 | 248;
+// 256 x 256 x 128 0.16 FP32 304 | 295, 0.49 389 | 403; 256 x 128 x 128 0.08
+// FP64 273 | 261, FP16s 90 | 87, 0.31 FP32 181 | 183, FP16s 114 | 123; on
+// fewer cells nothing to gain (128^3 FP32 0.02 74 | 74, 0.63 106 | 121).
+bool stage_by_list(bl_ibm g)
+{
+    const long n = g->lat->ncell;
+    return n >= 1l << 22 && g->NV * (n >= 1l << 23 ? 4 : 8) <= g->lat->ntiles;
+}
 
 // Velocity staging of the step whose binning is the last one.  Before that
 // binning's spreading (`spread` false) the last collision's force field and

@@ -8,7 +8,10 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 #   sides, cells of 642 vertices, the other staging
-CASES = [((131, 83, 101), 1, 1),    # few tiles of more than 2^20 cells: the list
+CASES = [((165, 159, 161), 1, 1),   # few tiles of more than 2^22 cells: the list
+         ((165, 159, 161), 13, 1),  # an eighth as many vertices as tiles: the list's last, one more: not
+         ((165, 159, 161), 14, 1),
+         ((131, 83, 101), 1, 1),    # few cells: a thread per cell
          ((101, 66, 103), 18, 0),   # most tiles of more than 96 MiB: the collision
          ((101, 66, 97), 18, 1)]    # the same a little below: a thread per cell
 
