@@ -386,9 +386,15 @@ __device__ __forceinline__ void touch_tile(int t, int* act, int* na, unsigned ch
 // vertex walking its tiles twice, with the weights stored (60 B a vertex in
 // FP32), took 16 us beside the element forces for 642 vertices and 99 us for
 // 400 800; this takes 7.1 and 87 us.
+// Vertices per lane group: one, and kBinMany from kManyVertices on, where
+// the chip is full and a workgroup of 256 vertices has fewer distinct tiles
+// per pair, so fewer global atomics.  Coupled steps, FP32, one | many: 10 272
+// vertices of 642-vertex cells 167 | 170 us, 20 544 188 | 188, 30 816 207 |
+// 201, 61 632 252 | 226; 46 224 in FP64 174 | 156; one mesh of 40 962, whose
+// numbering scatters, 159 | 164.
 constexpr int kBinLanes = 8;
-constexpr long kManyVertices = 65536;
-constexpr int kBinMany = 8;  // vertices per lane group from kManyVertices on: fewer distinct tiles per pair
+constexpr long kManyVertices = 24576;
+constexpr int kBinMany = 8;
 
 template <class R>
 struct BinArgs {
@@ -573,24 +579,19 @@ __device__ __forceinline__ void bin_body(long bx, const BinArgs<R>& A)
     }
 }
 
-// A binning workgroup of one vertex per lane group.
-template <class R>
-__device__ __forceinline__ void bin_one(long bx, const BinArgs<R>& A)
+// A binning workgroup of ITER vertices per lane group (with a boundary, one).
+template <class R, int ITER>
+__device__ __forceinline__ void bin_group(long bx, const BinArgs<R>& A)
 {
-    if (A.nw.on) bin_body<R, true, 1>(bx, A);
+    if (ITER > 1) bin_body<R, false, ITER>(bx, A);
+    else if (A.nw.on) bin_body<R, true, 1>(bx, A);
     else bin_body<R, false, 1>(bx, A);
 }
 
-template <class R>
+template <class R, int ITER>
 __global__ void __launch_bounds__(256) k_bin(BinArgs<R> a)
 {
-    bin_one<R>(ibm_block(blockIdx.x, gridDim.x, a.xcd), a);
-}
-
-template <class R>
-__global__ void __launch_bounds__(256) k_bin_many(BinArgs<R> a)
-{
-    bin_body<R, false, kBinMany>(ibm_block(blockIdx.x, gridDim.x, a.xcd), a);
+    bin_group<R, ITER>(ibm_block(blockIdx.x, gridDim.x, a.xcd), a);
 }
 
 __global__ void k_clear_bins(int* count, long n)
@@ -1629,11 +1630,11 @@ __global__ void __launch_bounds__(64 * kSpreadWaves) k_spread(SpreadArgs<R> a)
 // one launch: workgroups [0, n1) take the first, the others the second
 // (the choice is uniform over a workgroup, so its barriers stay whole).
 // Binning | element forces: both read the positions only.
-template <class R>
+template <class R, int ITER>
 __global__ void __launch_bounds__(256) k_bin_elem(BinArgs<R> b, int n1, ElemArgs<R> e)
 {
     const int bx = blockIdx.x;
-    if (bx < n1) bin_one<R>(ibm_block(bx, n1, b.xcd), b);
+    if (bx < n1) bin_group<R, ITER>(ibm_block(bx, n1, b.xcd), b);
     else elem_body<R>(ibm_block(bx - n1, (int)gridDim.x - n1, e.xcd), e);
 }
 
@@ -2287,6 +2288,8 @@ BinArgs<R> bin_args(bl_ibm g)
 // workgroups of a binning with bb threads each, iter vertices per lane group
 int bin_blocks(bl_ibm g, int bb, int iter) { return (int)nblk(g->NV, bb / kBinLanes * iter); }
 
+bool bin_many(bl_ibm g) { return g->NV >= kManyVertices && !g->has_boundary; }
+
 // host state after a binning has been enqueued
 void binned(bl_ibm g)
 {
@@ -2304,9 +2307,10 @@ int do_bin(bl_ibm g, hipStream_t s, hipEvent_t done = nullptr)
         with_vreal(g, [&](auto tag) {
             using R = decltype(tag);
             const int bb = g->lp[BL_IBM_BIN_BLOCK];
-            if (g->NV >= kManyVertices && !g->has_boundary)
-                hipLaunchKernelGGL(k_bin_many<R>, dim3(bin_blocks(g, bb, kBinMany)), dim3(bb), 0, s, bin_args<R>(g));
-            else hipLaunchKernelGGL(k_bin<R>, dim3(bin_blocks(g, bb, 1)), dim3(bb), 0, s, bin_args<R>(g));
+            if (bin_many(g))
+                hipLaunchKernelGGL((k_bin<R, kBinMany>), dim3(bin_blocks(g, bb, kBinMany)), dim3(bb), 0, s,
+                                   bin_args<R>(g));
+            else hipLaunchKernelGGL((k_bin<R, 1>), dim3(bin_blocks(g, bb, 1)), dim3(bb), 0, s, bin_args<R>(g));
             return 0;
         });
     if (done) BL_HIP(hipEventRecord(done, s));
@@ -2638,8 +2642,14 @@ int bin_elem_launch(bl_ibm g, hipStream_t s)
     with_vreal(g, [&](auto tag) {
         using R = decltype(tag);
         const int bb = g->lp[BL_IBM_BIN_BLOCK];  // both halves of the paired launch
-        const int nb = bin_blocks(g, bb, 1), ne = (int)nblk(g->NT + g->NP + g->NL, bb);
-        hipLaunchKernelGGL(k_bin_elem<R>, dim3(nb + ne), dim3(bb), 0, s, bin_args<R>(g), nb, elem_args<R>(g));
+        const bool many = bin_many(g);
+        const int nb = bin_blocks(g, bb, many ? kBinMany : 1), ne = (int)nblk(g->NT + g->NP + g->NL, bb);
+        if (many)
+            hipLaunchKernelGGL((k_bin_elem<R, kBinMany>), dim3(nb + ne), dim3(bb), 0, s, bin_args<R>(g), nb,
+                               elem_args<R>(g));
+        else
+            hipLaunchKernelGGL((k_bin_elem<R, 1>), dim3(nb + ne), dim3(bb), 0, s, bin_args<R>(g), nb,
+                               elem_args<R>(g));
         return 0;
     });
     BL_CHECK_LAUNCH();
@@ -3037,7 +3047,7 @@ __global__ void __launch_bounds__(256) k_bin_elem_batch(const LayeredEntry<R>* _
     const int box = batch_box(base, nbox, (int)blockIdx.x);
     const LayeredEntry<R>& E = tab[box];
     const int bx = (int)blockIdx.x - base[box];
-    if (bx < E.nb) bin_one<R>(ibm_block(bx, E.nb, E.bin.xcd), E.bin);
+    if (bx < E.nb) bin_group<R, 1>(ibm_block(bx, E.nb, E.bin.xcd), E.bin);
     else elem_body<R>(ibm_block(bx - E.nb, E.ne, E.elem.xcd), E.elem);
 }
 

@@ -106,3 +106,29 @@ def test_scattered_numbering_overflows_the_tile_table(device, kernel, storage):
         ib.close()
         L.close()
     assert np.array_equal(out[0], out[1])  # whatever order the atomics gave
+
+
+@pytest.mark.parametrize("storage", ["f64", "f32"])
+@pytest.mark.parametrize("cells", [9, 10])
+def test_paired_binning_below_and_above_its_line(device, cells, storage):
+    """One vertex a lane group (23 058) and eight (25 620) in the launch that
+    the binning shares with the element forces, against the stages one by one."""
+    from biblbm_amd import meshes
+    shape = (96, 92, 94)
+    centres = [(16.0 + 32 * (k % 3), 15.0 + 30 * (k // 3 % 3), 18.0 + 40 * (k // 9)) for k in range(cells)]
+    out = []
+    for paired in (True, False):
+        L, ib = _boundary("peskin", storage, shape, (1, 1, 1), meshes.icosphere(4, 11.0), centres)
+        start = ib.positions()
+        if paired:
+            ib.coupled_steps(6, use_graph=True)
+        else:
+            for _ in range(6):
+                ib.step()
+                L.collide_and_stream(1)
+        assert np.abs(ib.positions() - start).max() > 0
+        out.append((ib.positions(), ib.forces(), L.force()))
+        ib.close()
+        L.close()
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)  # the same sums in the same order
