@@ -957,7 +957,7 @@ struct StageArgs {
     LatView lv;
     const unsigned char* touched;
     void* ut;  // Vel4 of the storage's compute type
-    const int *active, *nactive;  // the touched-tile list
+    const int *active, *nactive;  // the touched-tile list (null: a thread per cell)
     FastDiv dty, dtz;             // division by the tiles along y and z
 };
 
@@ -1007,10 +1007,16 @@ __device__ __forceinline__ void stage_body(unsigned bx, unsigned nbx, const Stag
     if (A.touched[t]) stage_cell<S, SWAPPED>(A, c, x, y, z);
 }
 
-template <class S, bool SWAPPED, bool LIST>
+// Alone (k_gather_stage is the other launch) both forms stay in one kernel:
+// it then runs beside the membrane's on another stream, which lose more to
+// the cells' higher occupancy than the pass gains (256 x 128 x 128 FP64 with
+// 256 800 vertices and a phase field: 673 us a coupled step, 707 with the
+// forms apart).
+template <class S, bool SWAPPED>
 __global__ void __launch_bounds__(256) k_stage_u(StageArgs a)
 {
-    stage_body<S, SWAPPED, LIST>(blockIdx.x, gridDim.x, a);
+    if (a.active) stage_body<S, SWAPPED, true>(blockIdx.x, gridDim.x, a);
+    else stage_body<S, SWAPPED, false>(blockIdx.x, gridDim.x, a);
 }
 
 // ------------------------------------------------------- interpolation
@@ -2352,7 +2358,7 @@ StageArgs stage_args(bl_ibm g, bool spread)
     a.lv = ibm_view(g);
     a.touched = g->flags_alt;
     a.ut = g->ut;
-    a.active = g->active + (long)g->last_list * L->ntiles;
+    a.active = stage_by_list(g) ? g->active + (long)g->last_list * L->ntiles : nullptr;
     a.nactive = g->n_active + g->last_list;
     a.dty = make_fastdiv((unsigned)L->nty);
     a.dtz = make_fastdiv((unsigned)L->ntz);
@@ -2374,12 +2380,12 @@ unsigned stage_blocks(bl_ibm g, bool list)
 }
 
 template <class S>
-void launch_stage_s(const StageArgs& a, unsigned nblocks, bool swapped, bool list, hipStream_t s)
+void launch_stage_s(const StageArgs& a, unsigned nblocks, bool swapped, hipStream_t s)
 {
-    if (list && swapped) hipLaunchKernelGGL((k_stage_u<S, true, true>), dim3(nblocks), dim3(256), 0, s, a);
-    else if (list) hipLaunchKernelGGL((k_stage_u<S, false, true>), dim3(nblocks), dim3(256), 0, s, a);
-    else if (swapped) hipLaunchKernelGGL((k_stage_u<S, true, false>), dim3(nblocks), dim3(256), 0, s, a);
-    else hipLaunchKernelGGL((k_stage_u<S, false, false>), dim3(nblocks), dim3(256), 0, s, a);
+    if (swapped)
+        hipLaunchKernelGGL((k_stage_u<S, true>), dim3(nblocks), dim3(256), 0, s, a);
+    else
+        hipLaunchKernelGGL((k_stage_u<S, false>), dim3(nblocks), dim3(256), 0, s, a);
 }
 
 int launch_stage(bl_ibm g, hipStream_t s, bool spread)
@@ -2387,11 +2393,11 @@ int launch_stage(bl_ibm g, hipStream_t s, bool spread)
     bl_lattice L = g->lat;
     if (g->NV == 0) return BL_OK;
     const StageArgs a = stage_args(g, spread);
-    const bool swapped = (L->steps & 1) != 0, list = stage_by_list(g);
-    const unsigned nb = stage_blocks(g, list);
-    if (L->storage == BL_STORE_F64) launch_stage_s<double>(a, nb, swapped, list, s);
-    else if (L->storage == BL_STORE_F32) launch_stage_s<float>(a, nb, swapped, list, s);
-    else launch_stage_s<__half>(a, nb, swapped, list, s);
+    const bool swapped = (L->steps & 1) != 0;
+    const unsigned nb = stage_blocks(g, a.active != nullptr);
+    if (L->storage == BL_STORE_F64) launch_stage_s<double>(a, nb, swapped, s);
+    else if (L->storage == BL_STORE_F32) launch_stage_s<float>(a, nb, swapped, s);
+    else launch_stage_s<__half>(a, nb, swapped, s);
     BL_CHECK_LAUNCH();
     return BL_OK;
 }
