@@ -439,6 +439,13 @@ bool zseg_ok(const bl_lattice_s* L, int B)
            (size_t)Q * (size_t)L->stride <= 0xffffffffull;
 }
 
+static int force_mode(const bl_lattice_s* L)
+{
+    if (L->tile_flags && L->force_field) return 2;
+    if (L->g[0] != 0.0 || L->g[1] != 0.0 || L->g[2] != 0.0) return 1;
+    return 0;
+}
+
 // The launch shape of a lattice that nobody tuned, by the bytes of its
 // populations against the 256 MiB last-level cache (the pass is bound by
 // memory; 4 GiB copy on the same card: 6.17 TB/s).  Ratios are against one
@@ -457,7 +464,11 @@ bool zseg_ok(const bl_lattice_s* L, int B)
 //     x 257 1.00, 128 x 95 x 185 1.07; chunks on both parities 1.22, 0.97,
 //     1.01, 0.95, 0.98), but order 1 on both where planes start at multiples
 //     of 256 KiB and compete for the same sets (FP16s 672 x 192 x 64 0.92 in
-//     chunks, FP64 128^3 0.95, with hints 0.88).
+//     chunks, FP64 128^3 0.95, with hints 0.88).  With a force field, which
+//     a membrane's stages then use between the steps, FP64 and FP32 even
+//     steps stream past the cache in chunks of 16 here too (coupled steps
+//     with 3 | 40 cells: 128^3 FP64 143 | 202 -> 137 | 194 us, 161 x 165 x
+//     160 FP32 144 | 189 -> 136 | 177).
 //   beyond: chunks of 64 on both (FP16s 240 x 232 x 224 1.10, 375 MiB and
 //     more 1.00-1.16; FP32 204 x 200 x 181 1.11, 381 x 175 x 83 1.02; FP64
 //     301 x 129 x 181 1.04, 88 x 192 x 160 1.02).  Even steps of FP64 and FP32
@@ -487,7 +498,12 @@ void auto_launch(const bl_lattice_s* L, bool odd, bool emit, int& block, int& or
         return;
     }
     if (!emit && bytes <= kCache / 3 * 4) {
-        if (odd && plane % (256u << 10) != 0) order = 64;
+        const bool coupled = force_mode(L) == 2 && !half;
+        if (!odd && coupled) {
+            order = 16;
+            nt = 1;
+        }
+        if (odd && (coupled || plane % (256u << 10) != 0)) order = 64;
         return;
     }
     order = 64;
@@ -507,13 +523,6 @@ void auto_launch(const bl_lattice_s* L, bool odd, bool emit, int& block, int& or
         order = 16;
         nt = 1;
     }
-}
-
-static int force_mode(const bl_lattice_s* L)
-{
-    if (L->tile_flags && L->force_field) return 2;
-    if (L->g[0] != 0.0 || L->g[1] != 0.0 || L->g[2] != 0.0) return 1;
-    return 0;
 }
 
 CollidePlan collide_plan(const bl_lattice_s* L)

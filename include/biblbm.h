@@ -177,7 +177,7 @@ int bl_lattice_set_launch(bl_lattice lat, int block, int xcd_remap);
 int bl_lattice_set_launch_parity(bl_lattice lat, int parity, int block, int xcd_remap, int nontemporal);
 /* out = {block, xcd_remap, nontemporal} of one parity: as set, or, on a
  * lattice that no call fixed or tuned, what a plain collide-and-stream
- * takes by the lattice's size and storage. */
+ * takes by the lattice's size, storage and force field. */
 int bl_lattice_get_launch(bl_lattice lat, int parity, int out[3]);
 /* HIP stream the lattice works on (hipStream_t), for event timing. */
 int bl_lattice_stream(bl_lattice lat, void **stream);

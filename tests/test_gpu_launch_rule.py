@@ -46,6 +46,31 @@ def test_untuned_shapes_by_size(device, storage, shape, even, odd):
     assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
 
 
+@pytest.mark.parametrize("storage,shape,even,odd", [
+    ("f32", (128, 111, 124), (256, 1, 0), (256, 1, 0)),        # in the cache, as without
+    ("f64", (131, 128, 127), (256, 16, 1), (256, 64, 0)),      # up to 4/3 of it
+    ("f64", (128, 128, 128), (256, 16, 1), (256, 64, 0)),
+    ("f16s", (437, 128, 127), (256, 1, 0), (256, 64, 0)),
+])
+def test_untuned_shapes_with_a_force_field(device, storage, shape, even, odd):
+    from biblbm_amd.lattice import Lattice
+    rng = np.random.default_rng(4)
+    F = 1e-5 * rng.standard_normal(shape + (3,))
+    out = []
+    for fixed in (False, True):
+        L = Lattice(*shape, periodic=(1, 1, 1), storage=storage, omega=1.1)
+        L.set_force_field(F)
+        for p, want in ((0, even), (1, odd)):
+            assert tuple(L.launch(p).values()) == want
+        if fixed:
+            L.set_launch(256, True)
+        _state(L, np.random.default_rng(2))
+        L.collide_and_stream(3)
+        out.append(L.moments())
+        L.close()
+    assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
+
+
 @pytest.mark.parametrize("storage,n", [("f64", 128), ("f32", 154), ("f16s", 194)])
 def test_untuned_shapes_with_staging(device, storage, n):
     """Coupled steps beyond the cache with the velocity staging carried by
