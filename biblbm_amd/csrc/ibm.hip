@@ -297,6 +297,7 @@ constexpr int kProbes = 16;
 __device__ __forceinline__ int hash_insert(int* keys, int t)
 {
     unsigned h = ((unsigned)t * 2654435761u) >> (32 - kHashBits);
+#pragma unroll 1
     for (int probe = 0; probe < kProbes; ++probe) {
         const int old = atomicCAS(&keys[h], -1, t);
         if (old == -1 || old == t) return (int)h;
