@@ -983,13 +983,13 @@ __device__ __forceinline__ void stage_cell(const StageArgs& A, unsigned c, int x
     ((Vel4<C>*)A.ut)[c] = staged_velocity_m<FT, C>(lv, lv.flags, lv.force, m, c, x, y, z, j, invRho);
 }
 
-// LIST: off the touched-tile list.  At compile time: with both forms in one
-// kernel the cells' took 77 registers (FP64) where it takes 62 alone.
-template <class S, bool SWAPPED, bool LIST>
+// EITHER: off the touched-tile list where there is one; by cells only
+// otherwise.
+template <class S, bool SWAPPED, bool EITHER>
 __device__ __forceinline__ void stage_body(unsigned bx, unsigned nbx, const StageArgs& A)
 {
     const LatView& lv = A.lv;
-    if (LIST) {
+    if (EITHER && A.active) {
         const int na = *A.nactive, lane = threadIdx.x & 63;
         for (int a = (int)(bx * (blockDim.x >> 6) + (threadIdx.x >> 6)); a < na; a += (int)(nbx * (blockDim.x >> 6))) {
             const unsigned t = (unsigned)A.active[a], r = fdiv(t, A.dtz), tx = fdiv(r, A.dty);
@@ -1008,17 +1008,8 @@ __device__ __forceinline__ void stage_body(unsigned bx, unsigned nbx, const Stag
     if (A.touched[t]) stage_cell<S, SWAPPED>(A, c, x, y, z);
 }
 
-// Alone (k_gather_stage is the other launch) both forms stay in one kernel:
-// it then runs beside the membrane's on another stream, which lose more to
-// the cells' higher occupancy than the pass gains (256 x 128 x 128 FP64 with
-// 256 800 vertices and a phase field: 673 us a coupled step, 707 with the
-// forms apart).
 template <class S, bool SWAPPED>
-__global__ void __launch_bounds__(256) k_stage_u(StageArgs a)
-{
-    if (a.active) stage_body<S, SWAPPED, true>(blockIdx.x, gridDim.x, a);
-    else stage_body<S, SWAPPED, false>(blockIdx.x, gridDim.x, a);
-}
+__global__ void __launch_bounds__(256) k_stage_u(StageArgs a) { stage_body<S, SWAPPED, true>(blockIdx.x, gridDim.x, a); }
 
 // ------------------------------------------------------- interpolation
 // U_k = sum over the stencil nodes of phi(dx) phi(dy) phi(dz) u
@@ -1647,12 +1638,12 @@ __global__ void __launch_bounds__(256) k_bin_elem(BinArgs<R> b, int n1, ElemArgs
 
 // Vertex force gather (element forces) | velocity staging (the binning's
 // tiles, the last collision's field).
-template <class S, bool SWAPPED, bool LIST, class R, int GL>
+template <class S, bool SWAPPED, bool EITHER, class R, int GL>
 __global__ void __launch_bounds__(256) k_gather_stage(GatherArgs<R> ga, int n1, StageArgs sa)
 {
     const int bx = blockIdx.x;
     if (bx < n1) gather_body<R, GL>(ibm_block(bx, n1, ga.xcd), ga);
-    else stage_body<S, SWAPPED, LIST>(bx - n1, gridDim.x - n1, sa);
+    else stage_body<S, SWAPPED, EITHER>(bx - n1, gridDim.x - n1, sa);
 }
 
 // Spreading (lists, weights and vertex forces) | interpolation + advection
@@ -2893,23 +2884,31 @@ int step_fused(bl_ibm g)
 // The reference's order and every value are those of the other layouts;
 // no stage waits on another queue.
 // force gather (GL lanes per vertex) | velocity staging, one launch
-template <class S, bool LIST, class R, int GL>
-void launch_gather_stage_l(bl_ibm g, hipStream_t s)
+template <class S, bool EITHER, class R, int GL>
+void launch_gather_stage_of(bl_ibm g, hipStream_t s)
 {
     const int ng = (int)nblk(GL * g->NV);
     const StageArgs sa = stage_args(g, false);
-    const dim3 g2(ng + stage_blocks(g, LIST));
+    const dim3 g2(ng + stage_blocks(g, sa.active != nullptr));
     if (g->lat->steps & 1)
-        hipLaunchKernelGGL((k_gather_stage<S, true, LIST, R, GL>), g2, dim3(256), 0, s, gather_args<R>(g, true), ng, sa);
+        hipLaunchKernelGGL((k_gather_stage<S, true, EITHER, R, GL>), g2, dim3(256), 0, s, gather_args<R>(g, true), ng, sa);
     else
-        hipLaunchKernelGGL((k_gather_stage<S, false, LIST, R, GL>), g2, dim3(256), 0, s, gather_args<R>(g, true), ng, sa);
+        hipLaunchKernelGGL((k_gather_stage<S, false, EITHER, R, GL>), g2, dim3(256), 0, s, gather_args<R>(g, true), ng, sa);
 }
 
+// From 2^20 cells on by a kernel that has no list form: with it the cells'
+// form holds more registers, and 256 x 128 x 128 with 96 cells, FP16s, odd |
+// even steps, took 39.5 | 30.8 us, without 34.9 | 27.4.  Below, the kernel
+// with both is the shorter one (64^3 FP64 5.1 | 4.9 us, without 5.5 | 5.2).
+// k_stage_u, alone on its stream, keeps both: the membrane's kernels beside
+// it lose more to the cells' higher occupancy than it gains (256 x 128 x 128
+// FP64 with 256 800 vertices and a phase field: 676 us a coupled step, 707
+// without).
 template <class S, class R, int GL>
 void launch_gather_stage(bl_ibm g, hipStream_t s)
 {
-    if (stage_by_list(g)) launch_gather_stage_l<S, true, R, GL>(g, s);
-    else launch_gather_stage_l<S, false, R, GL>(g, s);
+    if (g->lat->ncell >= 1l << 20 && !stage_by_list(g)) launch_gather_stage_of<S, false, R, GL>(g, s);
+    else launch_gather_stage_of<S, true, R, GL>(g, s);
 }
 
 template <class S>
