@@ -464,8 +464,10 @@ __device__ __forceinline__ void place_pair(const BinArgs<R>& A, int code, int en
     if (slot < A.cap) A.list[(long)keys[sl] * A.cap + slot] = entry;
 }
 
-// ITER vertices per group of lanes, NEAR: a boundary is set (then ITER is 1
-// and a vertex's top-hat entry takes a second code).
+// ITER vertices per group of lanes, NEAR: a boundary is set (a near-wall
+// vertex's code carries kNearCode, and its top-hat entry takes a second one).
+constexpr int kNearCode = 1 << 30;
+
 template <class R, bool NEAR, int ITER>
 __device__ __forceinline__ void bin_body(long bx, const BinArgs<R>& A)
 {
@@ -473,7 +475,7 @@ __device__ __forceinline__ void bin_body(long bx, const BinArgs<R>& A)
     __shared__ int cnt[kHash];    // pairs per slot, then the run's first index in the tile's list
     __shared__ int fresh[kHash];  // tiles this workgroup reached first
     __shared__ int occ[kHash];    // occupied slots, compacted
-    __shared__ int codes[ITER > 1 ? ITER * 256 : 1];
+    __shared__ int codes[ITER > 1 ? (NEAR ? 2 : 1) * ITER * 256 : 1];
     __shared__ int n_fresh, n_pairs, fresh_base, n_occ;
     for (int i = threadIdx.x; i < kHash; i += blockDim.x) {
         keys[i] = -1;
@@ -502,7 +504,7 @@ __device__ __forceinline__ void bin_body(long bx, const BinArgs<R>& A)
             const long vn = min(v + vpw, A.NV - 1);
             for (int a = 0; a < 3; ++a) nx[a] = pos[3 * vn + a];
         }
-        code = e0 = -1;
+        code = codet = e0 = -1;
         if (v < A.NV) {
             // a vertex whose position is not finite (a membrane that blew
             // up) or absurdly far off touches no tile and is reported
@@ -537,7 +539,10 @@ __device__ __forceinline__ void bin_body(long bx, const BinArgs<R>& A)
                 code = count_pair(A, st, r, e0, keys, cnt, &n_pairs);
             }
         }
-        if (ITER > 1) codes[it * blockDim.x + threadIdx.x] = code;
+        if (ITER > 1) {
+            codes[it * blockDim.x + threadIdx.x] = code >= 0 && (e0 & kNearKey) ? code | kNearCode : code;
+            if (NEAR) codes[(ITER + it) * blockDim.x + threadIdx.x] = codet;
+        }
     }
     __syncthreads();
     // one global atomic per distinct tile; the occupied slots are compacted
@@ -566,8 +571,12 @@ __device__ __forceinline__ void bin_body(long bx, const BinArgs<R>& A)
     }
     if (ITER > 1) {
 #pragma unroll 4
-        for (int it = 0; it < ITER; ++it)
-            place_pair(A, codes[it * blockDim.x + threadIdx.x], (int)(v0 + it * vpw), keys, cnt);
+        for (int it = 0; it < ITER; ++it) {
+            const int v = (int)(v0 + it * vpw), c = codes[it * blockDim.x + threadIdx.x];
+            const bool nr = NEAR && c >= 0 && (c & kNearCode) != 0;
+            place_pair(A, nr ? c & ~kNearCode : c, nr ? kNearKey | (2 * v) : v, keys, cnt);
+            if (NEAR) place_pair(A, codes[(ITER + it) * blockDim.x + threadIdx.x], kNearKey | (2 * v + 1), keys, cnt);
+        }
     } else {
         place_pair(A, code, e0, keys, cnt);
         if (NEAR) place_pair(A, codet, e1, keys, cnt);
@@ -580,13 +589,12 @@ __device__ __forceinline__ void bin_body(long bx, const BinArgs<R>& A)
     }
 }
 
-// A binning workgroup of ITER vertices per lane group (with a boundary, one).
+// A binning workgroup of ITER vertices per lane group.
 template <class R, int ITER>
 __device__ __forceinline__ void bin_group(long bx, const BinArgs<R>& A)
 {
-    if (ITER > 1) bin_body<R, false, ITER>(bx, A);
-    else if (A.nw.on) bin_body<R, true, 1>(bx, A);
-    else bin_body<R, false, 1>(bx, A);
+    if (A.nw.on) bin_body<R, true, ITER>(bx, A);
+    else bin_body<R, false, ITER>(bx, A);
 }
 
 template <class R, int ITER>
@@ -2286,7 +2294,7 @@ BinArgs<R> bin_args(bl_ibm g)
 // workgroups of a binning with bb threads each, iter vertices per lane group
 int bin_blocks(bl_ibm g, int bb, int iter) { return (int)nblk(g->NV, bb / kBinLanes * iter); }
 
-bool bin_many(bl_ibm g) { return g->NV >= kManyVertices && !g->has_boundary; }
+bool bin_many(bl_ibm g) { return g->NV >= kManyVertices; }
 
 // host state after a binning has been enqueued
 void binned(bl_ibm g)

@@ -132,3 +132,31 @@ def test_paired_binning_below_and_above_its_line(device, cells, storage):
         L.close()
     for a, b in zip(*out):
         assert np.array_equal(a, b)  # the same sums in the same order
+
+
+@pytest.mark.parametrize("storage", ["f64", "f32"])
+@pytest.mark.parametrize("kernel", ["roma", "peskin"])
+@pytest.mark.parametrize("level", [5, 4])
+def test_many_vertices_near_a_wall(device, level, kernel, storage):
+    """Three membranes of 10 242 vertices (a lane group takes eight) and of
+    2 562 (one), some of them across the blend to the top hat at the plates."""
+    from biblbm_amd import meshes
+    from biblbm_amd.walls import Boundary
+    shape, per, plates = (60, 41, 56), (1, 0, 1), (0.5, 39.5)
+    centres = [(15.0, 14.9, 14.0), (44.0, 24.7, 15.0), (30.0, 20.0, 41.0)]
+    L, ib = _boundary(kernel, storage, shape, per, meshes.icosphere(level, 13.0), centres)
+    ib.set_boundary(Boundary.plates(*plates))
+    b = O.Boundary.plates(*plates)
+    pos = ib.positions()
+    assert pos[:, 1].min() < plates[0] + 1.4 and len(pos) == 3 * (10 * 4 ** level + 2)
+    ib.interpolate()
+    _, u = L.moments()
+    assert np.abs(ib.velocities() - O.interpolate_near(kernel, u, per, pos, b)).max() <= 64 * EPS[storage] * np.abs(u).max()
+    ib.compute_forces()
+    ib.spread()
+    f = ib.forces()
+    want = O.spread_near(kernel, shape, per, pos, f, b)
+    # as in _check; the blend weight, a distance of up to 20 less the half support, adds 20 units to each factor
+    assert np.abs(L.force() - want).max() <= 32 * EPS[storage] * np.abs(f).sum(0).max()
+    ib.close()
+    L.close()
