@@ -90,26 +90,32 @@ def test_untuned_shapes_with_staging(device, storage, n):
         assert np.array_equal(a, b)
 
 
-@pytest.mark.parametrize("storage", ["f64", "f32", "f16s"])
-def test_untuned_batches_by_size(device, storage):
-    """Batches below and beyond the cache against the hardware's order without hints."""
+@pytest.mark.parametrize("storage,sides,beyond", [
+    ("f64", (32, 48), False), ("f64", (96, 96, 96), True),
+    ("f32", (32, 48, 64), False), ("f32", (96,) * 4, True),
+    ("f16s", (96,) * 7, False), ("f16s", (96,) * 8, True),
+])
+def test_untuned_batches_by_size(device, storage, sides, beyond):
+    """Batches whose populations fit the 256 MiB cache and whose do not,
+    against another order and level of hints than the size gives them."""
     from biblbm_amd import workloads
     from biblbm_amd.ensemble import Ensemble
-    sides = (32,) if storage == "f64" else (96,) * (4 if storage == "f32" else 8)
-    for boxes in (sides, sides + (128,) * (1 if storage == "f64" else 0)):
-        out = []
-        for fixed in (False, True):
-            ws = [workloads.shear_box(storage, s, 0.9, 0.3, G=0.004, seed=k, radius=9.0 if s > 32 else 6.0)
-                  for k, s in enumerate(boxes)]
-            ens = Ensemble([(w.lattice, w.ibm) for w in ws])
-            if fixed:
-                ens.set_launch(0, 0, 0)
-                ens.set_launch(1, 0, 0)
-            ens.steps(4)
-            out.append([(w.ibm.positions(), w.lattice.moments()[1]) for w in ws])
-            ens.close()
-            for w in ws:
-                w.ibm.close()
-                w.lattice.close()
-        for a, b in zip(*out):
-            assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1])
+    size = {"f64": 8, "f32": 4, "f16s": 2}[storage]
+    assert (sum(19 * size * s ** 3 for s in sides) > 256 << 20) == beyond
+    out = []
+    for fixed in (False, True):
+        ws = [workloads.shear_box(storage, s, 0.9, 0.3, G=0.004, seed=k, radius=9.0 if s > 32 else 6.0)
+              for k, s in enumerate(sides)]
+        ens = Ensemble([(w.lattice, w.ibm) for w in ws])
+        if fixed:
+            for parity in (0, 1):
+                ens.set_launch(parity, *((0, 0) if beyond else (16, 1)))
+        ens.steps(4)
+        assert ens.batched
+        out.append([(w.ibm.positions(), w.lattice.moments()[1]) for w in ws])
+        ens.close()
+        for w in ws:
+            w.ibm.close()
+            w.lattice.close()
+    for a, b in zip(*out):
+        assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1])
