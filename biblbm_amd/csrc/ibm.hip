@@ -106,16 +106,6 @@ __device__ __forceinline__ V3<R> cross(V3<R> a, V3<R> b)
 template <class R>
 __device__ __forceinline__ R norm(V3<R> a) { return sqrt(dot(a, a)); }
 template <class R>
-struct Vec2;
-template <>
-struct Vec2<double> {
-    using T = double2;
-};
-template <>
-struct Vec2<float> {
-    using T = float2;
-};
-template <class R>
 __device__ __forceinline__ void st3(R* p, V3<R> a) { p[0] = a.x; p[1] = a.y; p[2] = a.z; }
 
 struct Grid {
@@ -400,7 +390,7 @@ constexpr int kBinMany = 8;
 template <class R>
 struct BinArgs {
     Grid gd;
-    int kernel, S;
+    int S;
     double h;
     long NV;
     const R* pos;
@@ -2269,7 +2259,6 @@ BinArgs<R> bin_args(bl_ibm g)
     bl_lattice L = g->lat;
     BinArgs<R> a;
     a.gd = grid_of(L);
-    a.kernel = g->kernel;
     a.S = g->S;
     a.h = g->h;
     a.NV = g->NV;
@@ -2347,11 +2336,10 @@ bool stage_by_list(bl_ibm g)
     return n >= 1l << 22 && g->NV * (n >= 1l << 23 ? 4 : 8) <= g->lat->ntiles;
 }
 
-// Velocity staging of the step whose binning is the last one.  Before that
-// binning's spreading (`spread` false) the last collision's force field and
-// flags are the lattice's, and the binning's flags are in flags_alt; after
-// it (`spread` true) the two have been swapped.
-StageArgs stage_args(bl_ibm g, bool spread)
+// Velocity staging of the step whose binning is the last one, before that
+// binning's spreading: the last collision's force field and flags are the
+// lattice's, and the binning's flags are in flags_alt.
+StageArgs stage_args(bl_ibm g)
 {
     bl_lattice L = g->lat;
     StageArgs a;
@@ -2362,11 +2350,6 @@ StageArgs stage_args(bl_ibm g, bool spread)
     a.nactive = g->n_active + g->last_list;
     a.dty = make_fastdiv((unsigned)L->nty);
     a.dtz = make_fastdiv((unsigned)L->ntz);
-    if (spread) {
-        a.lv.force = g->force_alt;
-        if (a.lv.flags) a.lv.flags = g->flags_alt;
-        a.touched = L->tile_flags;
-    }
     return a;
 }
 
@@ -2388,11 +2371,11 @@ void launch_stage_s(const StageArgs& a, unsigned nblocks, bool swapped, hipStrea
         hipLaunchKernelGGL((k_stage_u<S, false>), dim3(nblocks), dim3(256), 0, s, a);
 }
 
-int launch_stage(bl_ibm g, hipStream_t s, bool spread)
+int launch_stage(bl_ibm g, hipStream_t s)
 {
     bl_lattice L = g->lat;
     if (g->NV == 0) return BL_OK;
-    const StageArgs a = stage_args(g, spread);
+    const StageArgs a = stage_args(g);
     const bool swapped = (L->steps & 1) != 0;
     const unsigned nb = stage_blocks(g, a.active != nullptr);
     if (L->storage == BL_STORE_F64) launch_stage_s<double>(a, nb, swapped, s);
@@ -2567,7 +2550,7 @@ int do_interpolate(bl_ibm g)
 {
     int rc;
     if ((rc = do_bin(g, g->lat->stream))) return rc;
-    if ((rc = launch_stage(g, g->lat->stream, false))) return rc;
+    if ((rc = launch_stage(g, g->lat->stream))) return rc;
     return launch_interp(g, false, g->lat->stream);
 }
 
@@ -2748,7 +2731,7 @@ int step_serial(bl_ibm g)
     mark(g, 1);
     if ((rc = do_forces(g, s))) return rc;
     mark(g, 2);
-    if ((rc = launch_stage(g, s, false))) return rc;
+    if ((rc = launch_stage(g, s))) return rc;
     if (use_pairs(g)) {
         if ((rc = vreal_matches_storage(g))) return rc;
         const int st = g->lat->storage;
@@ -2793,7 +2776,7 @@ int step_forked(bl_ibm g)
     if ((rc = do_forces(g, A))) return rc;
     BL_HIP(hipEventRecord(e[1], A));
     if ((rc = do_bin(g, M, e[2]))) return rc;
-    if ((rc = launch_stage(g, M, false))) return rc;
+    if ((rc = launch_stage(g, M))) return rc;
     BL_HIP(hipStreamWaitEvent(A, e[2], 0));
     if ((rc = launch_spread(g, A))) return rc;
     BL_HIP(hipEventRecord(e[4], A));
@@ -2896,7 +2879,7 @@ template <class S, bool EITHER, class R, int GL>
 void launch_gather_stage_of(bl_ibm g, hipStream_t s)
 {
     const int ng = (int)nblk(GL * g->NV);
-    const StageArgs sa = stage_args(g, false);
+    const StageArgs sa = stage_args(g);
     const dim3 g2(ng + stage_blocks(g, sa.active != nullptr));
     if (g->lat->steps & 1)
         hipLaunchKernelGGL((k_gather_stage<S, true, EITHER, R, GL>), g2, dim3(256), 0, s, gather_args<R>(g, true), ng, sa);
@@ -3029,7 +3012,7 @@ int plan_layered(bl_ibm g, LayeredEntry<R>& E, int share)
     E.ne = (int)nblk(g->NT + g->NP + g->NL);
     binned(g);
     E.gather = gather_args<R>(g, true);
-    E.stage = stage_args(g, false);
+    E.stage = stage_args(g);
     E.ng = (int)nblk((long)g->lp[BL_IBM_GATHER_LANES] * g->NV);
     E.nst = (int)stage_blocks(g, false);  // a batch stages by cells
     unsigned nsp;
@@ -3130,7 +3113,7 @@ struct EnsembleBatch {
     int storage = 0, sw = 4, gl = 4;
     int order[2] = {0, 0};  // collide workgroup order per AA parity (collide_block modes)
     int nt[2] = {0, 0};     // and nontemporal level
-    bool any_ibm = false, any_vwall = false;
+    bool any_ibm = false;
     // velocity staging carried by the batched collision (every box has an
     // immersed boundary): no staging pass, the interpolation after the
     // collide-and-stream and the walls, as a single box's fused step
@@ -3330,7 +3313,6 @@ int ensemble_batch_build(const std::vector<bl_lattice>& lats, const std::vector<
                 vw.push_back(VwallPlan{view_of(L), L->nwall});
                 vcnt.push_back(vwall_blocks(L));
             }
-        B->any_vwall = !vw.empty();
         const size_t vtab = put(img, vw.data(), vw.size());
         st.vwall = put_launch(img, vtab, vcnt);
     }
@@ -3385,10 +3367,6 @@ void ensemble_batch_free(EnsembleBatch* B)
     hipFree(B->dev);
     delete B;
 }
-
-namespace {
-
-}  // namespace
 
 int ibm_step_launch(bl_ibm g, bool forked)
 {
