@@ -3,22 +3,25 @@
 // Per coupled step (the IBM functional of the reference,
 // src/fsi/DataProcessors.hh:94-108, preceded by the progs' computeVelocity
 // and force reset):
-//   bin      every vertex's delta-kernel stencil into 4x4x4 lattice tiles
-//            (counts, exclusive scan, list fill; atomics aggregated per
-//            workgroup in LDS);
+//   bin      every vertex's delta-kernel stencil into the lists of the 4x4x4
+//            lattice tiles it touches, in one pass (a workgroup counts its
+//            pairs per tile in LDS and reserves a run in each list), and a
+//            copy of its position;
 //   forces   per element (triangle / link / pair) contributions, then a
 //            per-vertex gather over the CSR incidence lists (K5, no atomics);
 //   stage    u = j/rho + F/2 on the cells of the touched tiles (from the
 //            post-stream populations and the force of the last collision);
-//   spread   one workgroup per touched tile: its vertex list is sorted in
-//            LDS, every cell sums g + sum_k phi F_k in vertex order (K6,
-//            deterministic, no float atomics);
-//   interp   U_k = sum phi phi phi u, one thread per vertex in the
-//            reference's node order (K4), fused with the advection x += U;
+//   spread   a wave per touched tile, a workgroup for a long list: the list
+//            put in vertex order, the tile's g + sum_k phi F_k a product of
+//            matrix instructions over it (K6, deterministic, no float
+//            atomics);
+//   interp   U_k = sum phi phi phi u, sixteen lanes per vertex (four for the
+//            top hat), each along x, and a butterfly (K4), fused with the
+//            advection x += U;
 //   move     per-particle area / volume / COM in FP64 with a
 //            fixed reduction order, COM mapped onto the periodic grid (K7);
-//   voxelize z-ray hits per column, sorted, parity fill of the phase (K8),
-//            only when the inner and outer viscosities differ.
+//   voxelize z-ray hits toggle a bit per column and node, parity fill of
+//            the phase (K8), only when the inner and outer viscosities differ.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -371,8 +374,8 @@ __device__ __forceinline__ void touch_tile(int t, int* act, int* na, unsigned ch
 // pairs are counted per distinct tile in LDS (the count at its insert is a
 // pair's place in the workgroup's run), one global atomic per tile reserves
 // the run.  The order within a list is whatever the atomics give; spreading
-// sorts.  The add that takes a tile past kSmallTile entries appends it to
-// the big-tile list.
+// sorts.  The add that takes a tile past BinArgs::small entries appends it
+// to the big-tile list.
 // Bound by latency on one cell and by instructions on many.  A thread per
 // vertex walking its tiles twice, with the weights stored (60 B a vertex in
 // FP32), took 16 us beside the element forces for 642 vertices and 99 us for
@@ -579,18 +582,24 @@ __device__ __forceinline__ void bin_body(long bx, const BinArgs<R>& A)
     }
 }
 
-// A binning workgroup of ITER vertices per lane group.
-template <class R, int ITER>
+// A binning workgroup: one vertex per lane group, or kBinMany.  MANY has its
+// two forms in kernels of their own: one kernel would hold the LDS of both
+// (400 800 vertices, FP32: 82 us alone, 125 together).
+enum BinForm { BIN_ONE, BIN_MANY, BIN_MANY_NEAR };
+
+template <class R, BinForm FORM>
 __device__ __forceinline__ void bin_group(long bx, const BinArgs<R>& A)
 {
-    if (A.nw.on) bin_body<R, true, ITER>(bx, A);
-    else bin_body<R, false, ITER>(bx, A);
+    if (FORM == BIN_MANY_NEAR) bin_body<R, true, kBinMany>(bx, A);
+    else if (FORM == BIN_MANY) bin_body<R, false, kBinMany>(bx, A);
+    else if (A.nw.on) bin_body<R, true, 1>(bx, A);
+    else bin_body<R, false, 1>(bx, A);
 }
 
-template <class R, int ITER>
+template <class R, BinForm FORM>
 __global__ void __launch_bounds__(256) k_bin(BinArgs<R> a)
 {
-    bin_group<R, ITER>(ibm_block(blockIdx.x, gridDim.x, a.xcd), a);
+    bin_group<R, FORM>(ibm_block(blockIdx.x, gridDim.x, a.xcd), a);
 }
 
 __global__ void k_clear_bins(int* count, long n)
@@ -639,8 +648,10 @@ struct ForceView {
 // (FP32) took 87 us when every quotient of the formulas was a division (67 of
 // them, about 12 instructions each) and takes 56.  So lengths are inverted
 // once, the three vertices share their scalar factors, and a force that is
-// minus the sum of the others is formed as that.  Against long double over
-// random triangles, pairs and links the errors are 0.85 to 1.0 of before.
+// minus the sum of the others is formed as that.  Errors of a cell's forces,
+// meshes of 162 to 2 562 vertices, against before: FP64 against long double
+// 0.87 to 0.99 (in-plane alone), 0.91 to 1.18 with the constraints, whose
+// error is that of the volume's sum; FP32 against FP64 0.85 to 1.01.
 
 // Skalak / NeoHookean in-plane forces of one triangle
 // (src/fsi/DeformableCapsule.hh:60-150), with the reference's
@@ -1198,8 +1209,10 @@ __global__ void __launch_bounds__(256) k_interp(InterpArgs<R> a)
 // the matrix instructions, 115 with one root per axis, the weights moved
 // to their cells by conditional shifts and the keys ranked, not sorted.
 // One launch (k_spread) holds two kinds of workgroups:
-//   small: tiles with at most kSmallTile entries (the touched-tile list,
-//          skipping the others), one wave per tile, four independent waves
+//   small: tiles with at most kSmallTile entries, kSparseTile where few
+//          tiles are touched (off the touched-tile list, or all of them in
+//          space order: spread_dense; the big ones are skipped), one wave
+//          per tile, four independent waves
 //          per workgroup, keys ranked against each other in LDS (up
 //          to 64 entries are loaded as listed and staged in the column of
 //          their rank, up to 128 put in order first), one running sum from
@@ -1626,11 +1639,11 @@ __global__ void __launch_bounds__(64 * kSpreadWaves) k_spread(SpreadArgs<R> a)
 // one launch: workgroups [0, n1) take the first, the others the second
 // (the choice is uniform over a workgroup, so its barriers stay whole).
 // Binning | element forces: both read the positions only.
-template <class R, int ITER>
+template <class R, BinForm FORM>
 __global__ void __launch_bounds__(256) k_bin_elem(BinArgs<R> b, int n1, ElemArgs<R> e)
 {
     const int bx = blockIdx.x;
-    if (bx < n1) bin_group<R, ITER>(ibm_block(bx, n1, b.xcd), b);
+    if (bx < n1) bin_group<R, FORM>(ibm_block(bx, n1, b.xcd), b);
     else elem_body<R>(ibm_block(bx - n1, (int)gridDim.x - n1, e.xcd), e);
 }
 
@@ -1644,9 +1657,9 @@ __global__ void __launch_bounds__(256) k_gather_stage(GatherArgs<R> ga, int n1, 
     else stage_body<S, SWAPPED, EITHER>(bx - n1, gridDim.x - n1, sa);
 }
 
-// Spreading (lists, weights and vertex forces) | interpolation + advection
-// (weights and staged velocity; it moves the vertices, which the spreading
-// does not read).
+// Spreading (lists, position copies and vertex forces) | interpolation +
+// advection (position copies and staged velocity; it moves the vertices,
+// which the spreading does not read).
 template <class S, int SW, class R>
 __global__ void __launch_bounds__(256) k_spread_interp(SpreadArgs<R> sp, int n1, InterpArgs<R> ia)
 {
@@ -1996,7 +2009,8 @@ __global__ void __launch_bounds__(256) k_ray_hits(ForceView<R> f, Grid gd, long 
 }
 // Fills kFillCols columns per workgroup, a lane per node (consecutive bytes),
 // and clears their bits for the next step.  `cap`: the most hits a step may
-// have.
+// have; more than 64 per triangle are those of a membrane torn far beyond
+// its lattice, and are reported.
 __global__ void __launch_bounds__(256) k_fill_columns(Grid gd, unsigned* bits, int* total, long cap, int* status,
                                                       unsigned char* phase)
 {
@@ -2280,10 +2294,21 @@ BinArgs<R> bin_args(bl_ibm g)
     return a;
 }
 
-// workgroups of a binning with bb threads each, iter vertices per lane group
-int bin_blocks(bl_ibm g, int bb, int iter) { return (int)nblk(g->NV, bb / kBinLanes * iter); }
+// workgroups of a binning with bb threads each
+int bin_blocks(bl_ibm g, int bb, bool many) { return (int)nblk(g->NV, bb / kBinLanes * (many ? kBinMany : 1)); }
 
 bool bin_many(bl_ibm g) { return g->NV >= kManyVertices; }
+
+// f(form, workgroups) with the boundary's form of binning
+template <class F>
+void with_bin_form(bl_ibm g, int bb, F f)
+{
+    const bool many = bin_many(g);
+    const int nb = bin_blocks(g, bb, many);
+    if (many && g->has_boundary && g->v_near) f(std::integral_constant<BinForm, BIN_MANY_NEAR>{}, nb);
+    else if (many) f(std::integral_constant<BinForm, BIN_MANY>{}, nb);
+    else f(std::integral_constant<BinForm, BIN_ONE>{}, nb);
+}
 
 // host state after a binning has been enqueued
 void binned(bl_ibm g)
@@ -2302,10 +2327,9 @@ int do_bin(bl_ibm g, hipStream_t s, hipEvent_t done = nullptr)
         with_vreal(g, [&](auto tag) {
             using R = decltype(tag);
             const int bb = g->lp[BL_IBM_BIN_BLOCK];
-            if (bin_many(g))
-                hipLaunchKernelGGL((k_bin<R, kBinMany>), dim3(bin_blocks(g, bb, kBinMany)), dim3(bb), 0, s,
-                                   bin_args<R>(g));
-            else hipLaunchKernelGGL((k_bin<R, 1>), dim3(bin_blocks(g, bb, 1)), dim3(bb), 0, s, bin_args<R>(g));
+            with_bin_form(g, bb, [&](auto form, int nb) {
+                hipLaunchKernelGGL((k_bin<R, decltype(form)::value>), dim3(nb), dim3(bb), 0, s, bin_args<R>(g));
+            });
             return 0;
         });
     if (done) BL_HIP(hipEventRecord(done, s));
@@ -2631,14 +2655,11 @@ int bin_elem_launch(bl_ibm g, hipStream_t s)
     with_vreal(g, [&](auto tag) {
         using R = decltype(tag);
         const int bb = g->lp[BL_IBM_BIN_BLOCK];  // both halves of the paired launch
-        const bool many = bin_many(g);
-        const int nb = bin_blocks(g, bb, many ? kBinMany : 1), ne = (int)nblk(g->NT + g->NP + g->NL, bb);
-        if (many)
-            hipLaunchKernelGGL((k_bin_elem<R, kBinMany>), dim3(nb + ne), dim3(bb), 0, s, bin_args<R>(g), nb,
-                               elem_args<R>(g));
-        else
-            hipLaunchKernelGGL((k_bin_elem<R, 1>), dim3(nb + ne), dim3(bb), 0, s, bin_args<R>(g), nb,
-                               elem_args<R>(g));
+        const int ne = (int)nblk(g->NT + g->NP + g->NL, bb);
+        with_bin_form(g, bb, [&](auto form, int nb) {
+            hipLaunchKernelGGL((k_bin_elem<R, decltype(form)::value>), dim3(nb + ne), dim3(bb), 0, s, bin_args<R>(g),
+                               nb, elem_args<R>(g));
+        });
         return 0;
     });
     BL_CHECK_LAUNCH();
@@ -2713,7 +2734,7 @@ int check_overflow(bl_ibm g)
     if (st[2] & 1)
         return fail(BL_ERR_CAPACITY, "immersed boundary: more than " + std::to_string(kTileCap) +
                                          " stencils touch one 4x4x4 tile");
-    if (st[2] & 2) return fail(BL_ERR_CAPACITY, "voxelization: hit buffer capacity exceeded");
+    if (st[2] & 2) return fail(BL_ERR_CAPACITY, "voxelization: more than 64 ray hits per triangle");
     if (st[2] & 4)
         return fail(BL_ERR_STATE, "immersed boundary: a vertex position is not finite (the membrane diverged)");
     return BL_OK;
@@ -3008,7 +3029,7 @@ int plan_layered(bl_ibm g, LayeredEntry<R>& E, int share)
     g->prepped = false;
     E.bin = bin_args<R>(g);
     E.elem = elem_args<R>(g);
-    E.nb = bin_blocks(g, 256, 1);
+    E.nb = bin_blocks(g, 256, false);
     E.ne = (int)nblk(g->NT + g->NP + g->NL);
     binned(g);
     E.gather = gather_args<R>(g, true);
@@ -3044,7 +3065,7 @@ __global__ void __launch_bounds__(256) k_bin_elem_batch(const LayeredEntry<R>* _
     const int box = batch_box(base, nbox, (int)blockIdx.x);
     const LayeredEntry<R>& E = tab[box];
     const int bx = (int)blockIdx.x - base[box];
-    if (bx < E.nb) bin_group<R, 1>(ibm_block(bx, E.nb, E.bin.xcd), E.bin);
+    if (bx < E.nb) bin_group<R, BIN_ONE>(ibm_block(bx, E.nb, E.bin.xcd), E.bin);
     else elem_body<R>(ibm_block(bx - E.nb, E.ne, E.elem.xcd), E.elem);
 }
 
