@@ -277,24 +277,26 @@ struct StencilTiles {
 // workgroup first aggregates its (tile, vertex) pairs in an LDS hash table
 // (open addressing, linear probing) and then issues one global atomic per
 // distinct tile.  A pair whose tile finds no slot within kProbes goes
-// straight to the global counter; counts stay exact either way.  256
-// neighbouring vertices touch a few dozen to two hundred tiles, so in 512
-// slots that is rare; 256 vertices scattered over a large membrane touch up
-// to 2 048, and there every further probe is spent for nothing (a
-// membrane of 40 962 vertices, FP32: 363 us a coupled step with 512 probes,
-// 164 with 16).
-constexpr int kHashBits = 9;
-constexpr int kHash = 1 << kHashBits;
+// straight to the global counter; counts stay exact either way.  A workgroup
+// of one vertex per lane group has at most 256 tiles (twice that near a
+// wall) and 2^9 slots.  One of eight, 256 neighbouring vertices, touches a
+// few dozen to some hundred, but 256 scattered over a large membrane up to
+// 2 048: 2^10 slots (132 x 111 x 124 suspension, FP64, 71 184 vertices in
+// meshes of 642 and 2 562: 282 us a coupled step with 2^9, 274), and no
+// more probes, which there are spent for nothing (one membrane of 40 962
+// vertices, FP32, 2^9 slots, in the many form: 363 us with 512 probes, 164
+// with 16; timed again, in a longer step, 217 with 64, 186 with 16).
 constexpr int kProbes = 16;
 
+template <int BITS>
 __device__ __forceinline__ int hash_insert(int* keys, int t)
 {
-    unsigned h = ((unsigned)t * 2654435761u) >> (32 - kHashBits);
+    unsigned h = ((unsigned)t * 2654435761u) >> (32 - BITS);
 #pragma unroll 1
     for (int probe = 0; probe < kProbes; ++probe) {
         const int old = atomicCAS(&keys[h], -1, t);
         if (old == -1 || old == t) return (int)h;
-        h = (h + 1) & (kHash - 1);
+        h = (h + 1) & ((1 << BITS) - 1);
     }
     return -1;
 }
@@ -422,7 +424,7 @@ __device__ __forceinline__ void put_pair(const BinArgs<R>& A, int t, int entry, 
 
 // This lane's tile of a stencil counted in the table: slot and rank there
 // (slot * 65536 + rank), or -1 when there is nothing left to place.
-template <class R>
+template <int BITS, class R>
 __device__ __forceinline__ int count_pair(const BinArgs<R>& A, const StencilTiles& st, int r, int entry, int* keys,
                                           int* cnt, int* n_pairs)
 {
@@ -432,7 +434,7 @@ __device__ __forceinline__ int count_pair(const BinArgs<R>& A, const StencilTile
     const int t = st.at2(A.gd, r >> 2, (r >> 1) & 1, r & 1);
     int code = -1;
     if (t >= 0) {
-        const int sl = hash_insert(keys, t);
+        const int sl = hash_insert<BITS>(keys, t);
         if (sl >= 0) code = (sl << 16) + atomicAdd(&cnt[sl], 1);
         else direct = t;
     }
@@ -464,6 +466,7 @@ constexpr int kNearCode = 1 << 30;
 template <class R, bool NEAR, int ITER>
 __device__ __forceinline__ void bin_body(long bx, const BinArgs<R>& A)
 {
+    constexpr int kBits = ITER > 1 ? 10 : 9, kHash = 1 << kBits;
     __shared__ int keys[kHash];
     __shared__ int cnt[kHash];    // pairs per slot, then the run's first index in the tile's list
     __shared__ int fresh[kHash];  // tiles this workgroup reached first
@@ -522,14 +525,14 @@ __device__ __forceinline__ void bin_body(long bx, const BinArgs<R>& A)
                         e1 = kNearKey | (int)(2 * v + 1);
                         StencilTiles stt;
                         stt.init(A.gd, 2, R(1.0), x);
-                        codet = count_pair(A, stt, r, e1, keys, cnt, &n_pairs);
+                        codet = count_pair<kBits>(A, stt, r, e1, keys, cnt, &n_pairs);
                     }
                 }
             }
             if (e0 >= 0) {
                 StencilTiles st;
                 st.init(A.gd, A.S, (R)A.h, x);
-                code = count_pair(A, st, r, e0, keys, cnt, &n_pairs);
+                code = count_pair<kBits>(A, st, r, e0, keys, cnt, &n_pairs);
             }
         }
         if (ITER > 1) {

@@ -92,7 +92,7 @@ def test_faces_cut_the_stencil(device, periodic, kernel, storage):
 @pytest.mark.parametrize("kernel", ["tophat", "peskin"])
 def test_scattered_numbering_overflows_the_tile_table(device, kernel, storage):
     """65 536 vertices or more are binned 256 a workgroup; numbered at random
-    they touch some 2 000 tiles, four times what the workgroup's table holds."""
+    they touch some 2 000 tiles, twice what the workgroup's table holds."""
     from biblbm_amd import meshes
     shape = (96, 92, 94)
     v, t = meshes.icosphere(6, 41.0)
