@@ -386,10 +386,13 @@ __device__ __forceinline__ void touch_tile(int t, int* act, int* na, unsigned ch
 // the chip is full and a workgroup of 256 vertices has fewer distinct tiles
 // per pair, so fewer global atomics.  Coupled steps, FP32, one | many: 10 272
 // vertices of 642-vertex cells 167 | 170 us, 20 544 188 | 188, 30 816 207 |
-// 201, 61 632 252 | 226; 46 224 in FP64 174 | 156; one mesh of 40 962, whose
-// numbering scatters, 159 | 164.
+// 201, 61 632 252 | 226; 46 224 in FP64 174 | 156.  A subdivided
+// sphere's numbering scatters the more the larger it is, so meshes above
+// kMeshVertices on average wait until kManyAny: one of 40 962 159 | 164, two
+// 284 | 271, eight of 10 242 376 | 350 (these three with 2^9 slots).  No
+// mesh between 10 242 and 40 962 was timed; the line lies in that gap.
 constexpr int kBinLanes = 8;
-constexpr long kManyVertices = 24576;
+constexpr long kManyVertices = 24576, kManyAny = 65536, kMeshVertices = 16384;
 constexpr int kBinMany = 8;
 
 template <class R>
@@ -2300,7 +2303,10 @@ BinArgs<R> bin_args(bl_ibm g)
 // workgroups of a binning with bb threads each
 int bin_blocks(bl_ibm g, int bb, bool many) { return (int)nblk(g->NV, bb / kBinLanes * (many ? kBinMany : 1)); }
 
-bool bin_many(bl_ibm g) { return g->NV >= kManyVertices; }
+bool bin_many(bl_ibm g)
+{
+    return g->NV >= kManyAny || (g->NV >= kManyVertices && g->NV <= kMeshVertices * g->np);
+}
 
 // f(form, workgroups) with the boundary's form of binning
 template <class F>
