@@ -3707,14 +3707,17 @@ int bl_ibm_init(bl_ibm g)
     if ((rc = vreal_upload(g, g->pos, 0, pos.data(), (long)pos.size(), L->stream))) return rc;
     g->ec_pair = 9 * g->NT;
     g->ec_link = g->ec_pair + 12 * g->NP;
+    // The clears below run on the lattice's stream, as what follows them does:
+    // it does not wait for the null stream, and a clear there may still be
+    // under way when the call returns.
     {
         const size_t csz = L->storage == BL_STORE_F64 ? sizeof(Vel4<double>) : sizeof(Vel4<float>);
         g->ut = nullptr;
         BL_HIP(hipMalloc(&g->ut, csz * (size_t)L->ncell));
-        BL_HIP(hipMemset(g->ut, 0, csz * (size_t)L->ncell));
+        BL_HIP(hipMemsetAsync(g->ut, 0, csz * (size_t)L->ncell, L->stream));
     }
-    BL_HIP(hipMemset(g->vel, 0, vr * 3 * std::max<long>(g->NV, 1)));
-    BL_HIP(hipMemset(g->force, 0, vr * 3 * std::max<long>(g->NV, 1)));
+    BL_HIP(hipMemsetAsync(g->vel, 0, vr * 3 * std::max<long>(g->NV, 1), L->stream));
+    BL_HIP(hipMemsetAsync(g->force, 0, vr * 3 * std::max<long>(g->NV, 1), L->stream));
     {  // vertex velocities and forces of particles loaded from a checkpoint
         long v0 = 0;
         for (const auto& p : g->parts) {
@@ -3730,11 +3733,11 @@ int bl_ibm_init(bl_ibm g)
     if ((rc = alloc(g->tile_count, L->ntiles)) || (rc = alloc(g->tile_list, (size_t)L->ntiles * kTileCap)) ||
         (rc = alloc(g->active, 4 * (size_t)L->ntiles)) || (rc = alloc(g->n_active, 16)))
         return rc;
-    BL_HIP(hipMemset(g->n_active, 0, 16 * sizeof(int)));
+    BL_HIP(hipMemsetAsync(g->n_active, 0, 16 * sizeof(int), L->stream));
     if ((rc = alloc(g->flags_alt, L->ntiles))) return rc;
-    BL_HIP(hipMemset(g->flags_alt, 0, L->ntiles));
+    BL_HIP(hipMemsetAsync(g->flags_alt, 0, L->ntiles, L->stream));
     BL_HIP(hipMalloc(&g->force_alt, 3 * L->stride * L->force_bytes));
-    BL_HIP(hipMemset(g->force_alt, 0, 3 * L->stride * L->force_bytes));
+    BL_HIP(hipMemsetAsync(g->force_alt, 0, 3 * L->stride * L->force_bytes, L->stream));
     {
         // chunks of 256 triangles per particle
         std::vector<int> choff{0}, tab, tvert;
@@ -3757,14 +3760,14 @@ int bl_ibm_init(bl_ibm g)
             (rc = alloc(g->ch_partial, kGeomSums * (size_t)std::max(g->nchunk, 1))))
             return rc;
     }
-    BL_HIP(hipMemset(g->tile_count, 0, L->ntiles * sizeof(int)));
+    BL_HIP(hipMemsetAsync(g->tile_count, 0, L->ntiles * sizeof(int), L->stream));
     // voxelization
     const size_t nbits = (size_t)L->nx * L->ny * column_words(L->nz);
     g->hit_cap = std::max<long>(64 * g->NT, 1024);
     if ((rc = alloc(g->col_bits, nbits)) || (rc = alloc(g->n_hits, 1)) || (rc = alloc(g->phase, L->ncell))) return rc;
-    BL_HIP(hipMemset(g->col_bits, 0, nbits * sizeof(unsigned)));
-    BL_HIP(hipMemset(g->n_hits, 0, sizeof(int)));
-    BL_HIP(hipMemset(g->phase, 0, L->ncell));
+    BL_HIP(hipMemsetAsync(g->col_bits, 0, nbits * sizeof(unsigned), L->stream));
+    BL_HIP(hipMemsetAsync(g->n_hits, 0, sizeof(int), L->stream));
+    BL_HIP(hipMemsetAsync(g->phase, 0, L->ncell, L->stream));
     for (auto& e : g->ev) BL_HIP(hipEventCreate(&e));
     for (auto& st : g->aux) BL_HIP(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
     for (auto& e : g->fev) BL_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
